@@ -24,7 +24,20 @@ struct LinFillArgs {
   // 2: one round at the threshold res[pid].pad, directions kept; the
   //    statistics of phase 1 are kept
   int phase;
+  // a fill that follows another one: the number of pairs the first left
+  // (their results say kLinLeft) and, for a fill that may leave some itself,
+  // its own count
+  const int* left_in = nullptr;
+  int* left_out = nullptr;
+  long long budget = 0;  // phase 2: the direction-store budget
+  int nd = 0;  // anti-diagonal fill in key form: bits of the delete count
 };
+
+// PairResult::full of a linear pair: 0 / 1 the stripe layout of a band / the
+// full plane, +2 the diagonal layout (linear_diag.hip); kLinLeft: not done,
+// handed to the next fill with the pending round's threshold in pad
+constexpr int kLinDiag = 2;
+constexpr int kLinLeft = -1;
 
 __device__ __forceinline__ int ldc8(const uint8_t* p, int j, int n) {
   return p[(unsigned)j < (unsigned)n ? j : 0];
@@ -43,6 +56,7 @@ __device__ __forceinline__ bool lin_full_plane(int L1, int L2, int deltawh) {
 
 template <bool kDm>
 __global__ __launch_bounds__(64) void k_linear_fill(LinFillArgs A) {
+  if (A.left_in && *A.left_in == 0) return;
   __shared__ int s_cost[1024];
   __shared__ int s_prep[32];
   __shared__ int s_tail[32];
@@ -59,6 +73,7 @@ __global__ __launch_bounds__(64) void k_linear_fill(LinFillArgs A) {
     const int q = wave_grab(A.counter);
     if (q >= A.pt.n) break;
     const int pid = A.pt.order[q];
+    if (A.left_in && A.res[pid].full != kLinLeft) continue;
     const uint8_t* __restrict__ sa = A.pt.blob + rows_off(A.pt, pid);
     const uint8_t* __restrict__ sb = A.pt.blob + cols_off(A.pt, pid);
     const int L1 = A.pt.len_a[pid], L2 = A.pt.len_b[pid];
@@ -78,6 +93,12 @@ __global__ __launch_bounds__(64) void k_linear_fill(LinFillArgs A) {
       T = r1.pad;
       rounds = r1.rounds - 1;
       cells1 = r1.cells;
+      slots = lane == 0 ? r1.slots : 0;
+    } else if (A.left_in) {
+      const PairResult r1 = A.res[pid];
+      T = r1.pad;
+      rounds = r1.rounds;
+      cells = lane == 0 ? r1.cells : 0;
       slots = lane == 0 ? r1.slots : 0;
     }
     int Tfin = T;
@@ -320,8 +341,8 @@ __global__ __launch_bounds__(64) void k_linear_backtrace(LinBtArgs A) {
   const uint8_t* dm = A.dm + A.pt.dm_off[pid];
   const long long* stab = A.stab + A.pt.stab_off[pid];
   const PairResult R = A.res[pid];
-  const bool full = R.full != 0;
-  const int newk = R.newk;
+  const bool full = (R.full & 1) != 0;
+  const int newk = __builtin_amdgcn_readfirstlane(R.newk);
   const long long dm_cap = lin_dm_bytes(L1, L2);
 
   // ---- walk ----------------------------------------------------------------
@@ -340,6 +361,72 @@ __global__ __launch_bounds__(64) void k_linear_backtrace(LinBtArgs A) {
   const int top_b = A.lim ? A.lim_st2 + A.lim_a2 - 1 : L2 - 1;
   int cb = -1, jlo = 0;
   long long base = 0;  // first 16-step block of the stripe
+  if (__builtin_amdgcn_readfirstlane(R.full) & kLinDiag) {
+    // diagonal layout: a run of diagonal moves stays in one slot's words,
+    // its cells 4 bits apart, so each turn takes the diagonal moves down to
+    // the next up or left move of the word (or to the word's start)
+    const int stride = diag_stride(L2 - L1, newk);
+    const int newke = (newk + 1) & ~1;
+    // the round's words (counted in 256-byte lines of the pair's region)
+    const unsigned* const dw =
+        reinterpret_cast<const unsigned*>(dm) +
+        ((long long)__builtin_amdgcn_readfirstlane((int)stab[0]) << 6);
+    int wq = -(1 << 28), wc = 0;  // the window: blocks wq .. wq - 3, slots wc .. wc + 63
+    int nq = -(1 << 28), nc = 0;  // the next one, loading behind it
+    auto word = [&](int q, int c0) __attribute__((always_inline)) -> uint32_t {
+      const int c = c0 + lane;
+      return (q >= 0 && (unsigned)c < (unsigned)stride) ? dw[(long long)q * stride + c] : 0u;
+    };
+    while (i > 0 && j > 0) {
+      const int q = (i + j) >> 4, u = (i + j) & 15;
+      const int c = (j - i + newke) >> 1;
+      if (q > wq || q < wq - 3 || c < wc || c >= wc + 64) {
+        if (q <= nq && q >= nq - 3 && c >= nc && c < nc + 64) {
+          wa0 = wb0; wa1 = wb1; wa2 = wb2; wa3 = wb3;
+          wq = nq;
+          wc = nc;
+        } else {
+          wq = q;
+          wc = c - 32;
+          wa0 = word(q, wc);
+          wa1 = word(q - 1, wc);
+          wa2 = word(q - 2, wc);
+          wa3 = word(q - 3, wc);
+        }
+        nq = wq - 4;
+        nc = c - 32;
+        wb0 = word(nq, nc);
+        wb1 = word(nq - 1, nc);
+        wb2 = word(nq - 2, nc);
+        wb3 = word(nq - 3, nc);
+      }
+      const int k = wq - q;
+      const uint32_t v = k < 2 ? (k == 0 ? wa0 : wa1) : (k == 2 ? wa2 : wa3);
+      const uint32_t w = __builtin_amdgcn_readlane(v, c - wc);
+      // the moves of this diagonal's cells at and below this step
+      const uint32_t t = w & ((u & 1) ? 0x88888888u : 0x22222222u) & (0xFFFFFFFFu >> (30 - 2 * u));
+      const int hit = t ? (31 - __builtin_clz(t)) >> 1 : -1;
+      int run = t ? (u - hit) >> 1 : (u >> 1) + 1;
+      const int m = imin(i, j);
+      const bool ends = run >= m;
+      if (ends) run = m;
+      i -= run;
+      j -= run;
+      const int n1 = n + run;
+      if ((n ^ n1) >> 6) {  // at most 8 moves: one chunk boundary
+        r1[cap - 1 - ((n1 & ~63) - 64) - lane] = (uint8_t)mv;
+        mv = 0;
+      }
+      n = n1;
+      if (t && !ends) {
+        const int code = ((w >> (2 * hit)) & 1) ? 1 : 2;
+        record(code);
+        if ((n & 63) == 0) mv = 0;
+        if (code == 1) i--;
+        else j--;
+      }
+    }
+  }
   while (i > 0 && j > 0) {
     const int bb = (i - 1) >> 6;
     if (bb != cb) {

@@ -125,6 +125,14 @@ __device__ __forceinline__ void lin_mw_pair(MwShared<NW>& S, const LinFillArgs& 
       rounds = r1.rounds - 1;
       cells1 = r1.cells;
       slots1 = r1.slots;
+    } else if (A.left_in) {
+      const PairResult r1 = A.res[pid];
+      T = r1.pad;
+      rounds = r1.rounds;
+      if (tid == 0) {
+        cells = r1.cells;
+        slots = r1.slots;
+      }
     }
     int Tfin = T;
     for (;;) {
@@ -491,6 +499,7 @@ template <bool kDm, bool kDc, int NW>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4))) void k_linear_mw(LinFillArgs A) {
   __shared__ MwShared<NW> S;
   const int tid = threadIdx.x;
+  if (A.left_in && *A.left_in == 0) return;
   for (int k = tid; k < 1024; k += 64 * NW) {
     const int c = A.cm->cost[k];
     S.cost[k] = c;
@@ -509,6 +518,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4))) vo
     __syncthreads();  // the next grab rewrites S.pair
     if (q >= A.pt.n) break;
     const int pid = A.pt.order[q];
+    if (A.left_in && A.res[pid].full != kLinLeft) continue;
     if (A.pt.prio[pid])
       lin_mw_pair<kDm, kDc, true, NW>(S, A, pid, ring0);
     else

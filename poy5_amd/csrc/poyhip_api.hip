@@ -25,6 +25,7 @@
 #include "cube_mw.hip"
 #include "linear.hip"
 #include "linear_mw.hip"
+#include "linear_diag.hip"
 #include "medians.hip"
 #include "newkk.hip"
 #include "unions.hip"
@@ -99,6 +100,13 @@ struct poyhip_ctx {
   // wavefronts of its own pairs; 1: a workgroup per pair; 0: a wavefront
   int lin_wg = 2;
   bool lin_fits = false;
+  // largest entry of the 5-bit cost, prepend and tail tables, -1 when an
+  // entry is negative (the anti-diagonal linear fill bounds its sums below
+  // the value it marks cells outside the band with)
+  int lin_max = -1;
+  // some symbol's tail cost is below its deletion cost (the last column then
+  // has a rule of its own, which the key form of that fill leaves out)
+  bool lin_tails = false;
   // largest entry of the 3D cost table, -1 when an entry is negative (the
   // workgroup fill carries 8*value + code keys and needs values below 2^27)
   int cm3_max = -1;
@@ -216,7 +224,8 @@ bool valid_seq(const uint8_t* s, int l) {
 // Offsets of the one-pair descriptor block used by the drop-in calls.
 struct OneDesc {
   int64_t off1, off2, dm_off, stab_off, out_off;
-  int len_a, len_b, swapped, prio, deltawh, order, counter, pad;
+  int len_a, len_b, swapped, prio, deltawh, order;
+  int counter[8];  // work counters of the launches, zero (kLinCounters)
 };
 constexpr size_t kDescBytes = 128;
 static_assert(sizeof(OneDesc) <= kDescBytes, "descriptor block");
@@ -264,7 +273,7 @@ int stage_pair(poyhip_ctx* c, const uint8_t* a, int la, const uint8_t* b, int lb
   memcpy(c->h_stage.data() + kDescBytes + la, b, lb);
   HIPCHK(c, hipMemcpyAsync(c->stage.p, c->h_stage.data(), need, hipMemcpyHostToDevice, c->stream));
   *t = one_table(c->stage.p, static_cast<const uint8_t*>(c->stage.p) + kDescBytes);
-  *counter = &reinterpret_cast<OneDesc*>(c->stage.p)->counter;
+  *counter = reinterpret_cast<OneDesc*>(c->stage.p)->counter;
   return POYHIP_OK;
 }
 
@@ -339,18 +348,101 @@ int64_t lin_ws_slot_ints(int Lb) {
   return std::max(lin_ws_ints(Lb), lin_mw_ws_ints(Lb, kLinMwWaves));
 }
 
-// Launches the linear fill of A.pt.n pairs: the multi-wavefront kernel (one
-// workgroup per pair) when the context's table allows it, else the
-// wavefront-per-pair kernel.  `slots` workspace slots of A.ws_stride ints
-// are available.  Returns the kernel's launch error.
-hipError_t launch_linear_fill(poyhip_ctx* c, const LinFillArgs& A, bool dm, int slots,
-                              hipStream_t st) {
+// Work counters of one linear fill: its queue and the count of the pairs it
+// left, of the anti-diagonal fills in turn, then the queue of the stripe fill.
+constexpr int kLinCounters = 8;
+
+// The anti-diagonal fill takes a launch whose costs fit its records and
+// whose sums stay below its out-of-band mark.
+bool lin_diag_ok(const poyhip_ctx* c, int64_t max_sum) {
+  return c->lin_wg == 2 && c->lin_fits && c->lin_max >= 0 &&
+         (max_sum + 2) * (int64_t)c->lin_max < ((int64_t)1 << 29);
+}
+
+// Bits of a delete count when value and count share a 32-bit key (L1 is at
+// most half of max_sum), 0 when they do not fit.
+int lin_key_bits(const poyhip_ctx* c, int64_t max_sum) {
+  int nd = 1;
+  while (((int64_t)1 << nd) <= max_sum / 2 + 1) nd++;
+  const bool fits = !c->lin_tails && nd <= 16 &&
+                    (max_sum + 2) * std::max(c->lin_max, 1) < ((int64_t)1 << (29 - nd));
+  return fits ? nd : 0;
+}
+
+template <int NW>
+void launch_linear_key(const LinFillArgs& A, bool dm, int grid, hipStream_t st) {
+  if (dm)
+    hipLaunchKernelGGL((k_linear_diag<NW, true, true, true>), dim3(grid), dim3(64 * NW), 0, st, A);
+  else
+    hipLaunchKernelGGL((k_linear_diag<NW, true, false, true>), dim3(grid), dim3(64 * NW), 0, st, A);
+}
+
+void launch_linear_wide(const LinFillArgs& A, bool dm, int grid, hipStream_t st) {
+  // phase 2 needs no delete counts: its rounds are known
+  const dim3 blk(64 * 16);
+  if (A.phase == 2)
+    hipLaunchKernelGGL((k_linear_diag<16, false, true, false>), dim3(grid), blk, 0, st, A);
+  else if (dm)
+    hipLaunchKernelGGL((k_linear_diag<16, false, true, true>), dim3(grid), blk, 0, st, A);
+  else
+    hipLaunchKernelGGL((k_linear_diag<16, false, false, true>), dim3(grid), blk, 0, st, A);
+}
+
+// Launches the linear fill of A.pt.n pairs, A.counter[0 .. kLinCounters) zero.
+// `max_sum` is the largest L1 + L2 of the launch, `slots` workspace slots of
+// A.ws_stride ints are available.  `diag` false keeps to the stripe fills.
+// Returns the launch error.
+//
+// The anti-diagonal fill comes first: in key form with one wavefront per pair
+// when the pairs alone fill the SIMDs, four when they do not and sixteen when
+// every pair can have a CU, in wide form with sixteen when value and count do
+// not fit a key.  Pairs it leaves (a
+// band wider than its lanes, a direction store larger than the stripe
+// layout's region) go through the sixteen-wavefront form, then the stripe
+// fill.
+hipError_t launch_linear_fill(poyhip_ctx* c, const LinFillArgs& A0, bool dm, int slots,
+                              int64_t max_sum, bool diag, hipStream_t st) {
+  LinFillArgs A = A0;
   const int n = A.pt.n;
+  int* const cnt = A.counter;
+  if (diag && lin_diag_ok(c, max_sum)) {
+    const int max_band = (int)std::min<int64_t>(max_sum, INT_MAX);
+    const int wide_grid = std::max(1, std::min(n, c->num_cus));
+    A.left_out = cnt + 1;
+    A.nd = lin_key_bits(c, max_sum);
+    int cap = DiagGeom<8, 16>::kMaxBand;
+    if (!A.nd) {
+      launch_linear_wide(A, dm, wide_grid, st);
+    } else if (n <= c->num_cus) {
+      launch_linear_key<16>(A, dm, wide_grid, st);
+    } else if (n > 6 * c->num_cus) {
+      launch_linear_key<1>(A, dm, std::max(1, std::min(n, c->num_cus * c->waves_per_cu)), st);
+      cap = DiagGeom<8, 1>::kMaxBand;
+    } else {
+      launch_linear_key<4>(A, dm, std::max(1, std::min(n, c->num_cus * 4)), st);
+      cap = DiagGeom<8, 4>::kMaxBand;
+    }
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    if (max_band > cap && cap < DiagGeom<8, 16>::kMaxBand) {
+      A.left_in = cnt + 1;
+      A.left_out = cnt + 3;
+      A.counter = cnt + 2;
+      launch_linear_wide(A, dm, wide_grid, st);
+      e = hipGetLastError();
+      if (e != hipSuccess) return e;
+      cap = DiagGeom<8, 16>::kMaxBand;
+    }
+    if (!dm && max_band <= cap) return hipSuccess;
+    A.left_in = A.left_out;
+    A.left_out = nullptr;
+    A.counter = cnt + 4;
+  }
   // with four of its own pairs per SIMD a batch keeps the device busy with
   // one wavefront per pair, which saves the workgroup's block barriers and
   // stripe schedule (a level of ~600-symbol pairs runs ~1.5x faster); the
   // workgroup pays off when fewer, longer pairs must fill the device
-  const bool mw = c->lin_mw && (c->lin_wg == 1 || n < 16 * c->num_cus);
+  const bool mw = c->lin_mw && (c->lin_wg == 1 || A.left_in || n < 16 * c->num_cus);
   if (mw) {
     const int grid = std::max(1, std::min({n, slots, c->num_cus * kLinMwPerCu}));
     const dim3 blk(64 * kLinMwWaves);
@@ -396,7 +488,9 @@ int run_linear_one(poyhip_ctx* c, const uint8_t* s1, int l1, const uint8_t* s2, 
   A.res = dres;
   A.counter = counter;
   A.phase = 0;
-  HIPCHK(c, launch_linear_fill(c, A, true, 1, c->stream));
+  // a limited walk may start outside the band, where only the stripe layout
+  // says what it reads
+  HIPCHK(c, launch_linear_fill(c, A, true, 1, (int64_t)l1 + l2, limit == nullptr, c->stream));
   size_t back = sizeof(PairResult);
   if (backtrace) {
     LinBtArgs B;
@@ -638,6 +732,13 @@ int poyhip_set_cm(poyhip_ctx* c, const poyhip_cm* cm) {
     mx = std::max(mx, cm->cost[k]);
   }
   c->cm_max = neg ? -1 : mx;
+  for (int k = 0; k < 32; k++) {
+    neg |= cm->prepend[k] < 0 || cm->tail[k] < 0;
+    mx = std::max({mx, cm->prepend[k], cm->tail[k]});
+  }
+  c->lin_max = neg ? -1 : mx;
+  c->lin_tails = false;
+  for (int k = 1; k < 32; k++) c->lin_tails |= cm->tail[k] < cm->cost[(k << 5) + 16];
   return POYHIP_OK;
 }
 
@@ -1029,7 +1130,7 @@ int poyhip_align_affine_3_noalloc(poyhip_ctx* c, const uint8_t* si, int li, cons
   A.ws_stride = 0;
   A.stab = reinterpret_cast<long long*>(S + L.stab);
   A.res = dres;
-  A.counter = &reinterpret_cast<OneDesc*>(S)->counter;
+  A.counter = reinterpret_cast<OneDesc*>(S)->counter;
   A.cls = nullptr;
   A.ngen = nullptr;
   int any = 0;
@@ -1214,6 +1315,7 @@ struct poyhip_batch {
   // diagonal-store batches: some pair's longer sequence reaches 2^16 (both
   // 16-bit gap counts carried)
   bool wide = false;
+  int64_t max_sum = 0;  // largest L1 + L2
   std::vector<PairResult> h_res;
   // graph replay
   bool use_graph = false;
@@ -1276,6 +1378,15 @@ int64_t lin_dm_exact(int L1, int L2, int newk, bool full) {
   return tot;
 }
 
+// Region of a linear pair in phase 2: its final band in the stripe layout, or
+// in the diagonal layout where the anti-diagonal fill takes it.
+int64_t lin_region_bytes(int L1, int L2, int newk, bool full, int64_t budget) {
+  const int64_t stripes = lin_dm_exact(L1, L2, newk, full);
+  if (L1 < 2 || diag_slots(L2 - L1, newk) > 8 * DiagGeom<8, 16>::kLanes) return stripes;
+  const int64_t diag = diag_dm_bytes(L1, L2, newk);
+  return diag <= budget ? std::max(stripes, diag) : stripes;
+}
+
 void batch_free_device(poyhip_batch* b) {
   for (void* p : {(void*)b->d_tab, (void*)b->d_res, (void*)b->d_dm, (void*)b->d_ws,
                   (void*)b->d_stab, (void*)b->d_counters, (void*)b->d_cls})
@@ -1322,9 +1433,9 @@ int batch_enqueue(poyhip_batch* b, const uint8_t* blob, const int64_t* off1, con
   const int nch = (int)b->chunks.size();
   if (timing) HIPCHK(c, hipEventRecord(b->ev[2 * nch], st));
   // counters: two per chunk (fast and general fill queues), then the number
-  // of general-class pairs
-  hipLaunchKernelGGL(k_zero_ints, dim3((2 * nch + 1 + 63) / 64), dim3(64), 0, st, b->d_counters,
-                     2 * nch + 1);
+  // of general-class pairs; a linear fill's own set per chunk
+  const int nzero = op_is_linear(b->op) ? kLinCounters * nch : 2 * nch + 1;
+  hipLaunchKernelGGL(k_zero_ints, dim3((nzero + 63) / 64), dim3(64), 0, st, b->d_counters, nzero);
   if (b->op == POYHIP_OP_ALIGN_AFFINE) {
     PairTable all = batch_table(b, blob, off1, off2, -1);
     hipLaunchKernelGGL(k_affine_classify, dim3(b->n), dim3(64), 0, st, all, b->d_cls,
@@ -1402,9 +1513,9 @@ int batch_enqueue(poyhip_batch* b, const uint8_t* blob, const int64_t* off1, con
         A.ws_stride = b->ws_stride;
         A.stab = b->d_stab;
         A.res = b->d_res;
-        A.counter = b->d_counters + k;
+        A.counter = b->d_counters + kLinCounters * k;
         A.phase = 0;
-        HIPCHK(c, launch_linear_fill(c, A, b->op == POYHIP_OP_ALIGN_2D, b->grid, st));
+        HIPCHK(c, launch_linear_fill(c, A, b->op == POYHIP_OP_ALIGN_2D, b->grid, b->max_sum, true, st));
       }
     }
     HIPCHK(c, hipGetLastError());
@@ -1477,6 +1588,7 @@ int poyhip_batch_create(poyhip_ctx* c, int op, int n, const int* len1, const int
     b->la[k] = sw ? len2[k] : len1[k];
     b->lb[k] = sw ? len1[k] : len2[k];
     maxlb = std::max(maxlb, b->lb[k]);
+    b->max_sum = std::max(b->max_sum, (int64_t)b->la[k] + b->lb[k]);
     work[k] = (double)b->la[k] * (double)b->lb[k];
     if (op_is_newkk(op)) {
       const int rc = nk_check(c, b->la[k], b->lb[k]);
@@ -1560,7 +1672,8 @@ int poyhip_batch_create(poyhip_ctx* c, int op, int n, const int* len1, const int
   b->d_order = reinterpret_cast<int*>(p); p += 4 * (size_t)n;
   if (ctx_malloc(c, (void**)&b->d_res, sizeof(PairResult) * (size_t)n) != hipSuccess)
     return fail(POYHIP_ENOMEM, "results");
-  const size_t ncounters = b->two_phase ? 2 * (size_t)n + 4 : 2 * b->chunks.size() + 2;
+  const size_t per = op_is_linear(op) ? kLinCounters : 2;
+  const size_t ncounters = b->two_phase ? per * ((size_t)n + 2) : per * b->chunks.size() + 2;
   if (ctx_malloc(c, (void**)&b->d_counters, sizeof(int) * ncounters) != hipSuccess)
     return fail(POYHIP_ENOMEM, "counters");
   if (ctx_malloc(c, (void**)&b->d_cls, (size_t)n + 64) != hipSuccess) return fail(POYHIP_ENOMEM, "classes");
@@ -1694,10 +1807,13 @@ int batch_run_two_phase(poyhip_batch* b, const uint8_t* d_blob, const int64_t* d
     ~EvGuard() { for (auto e : *v) (void)hipEventDestroy(e); }
   } guard{&ev};
   HIPCHK(c, hipEventRecord(ev[0], st));
-  hipLaunchKernelGGL(k_zero_ints, dim3((2 * n + 4 + 255) / 256), dim3(256), 0, st, b->d_counters,
-                     2 * n + 4);
-  PairTable all = batch_table(b, d_blob, d_off1, d_off2, -1);
+  // counters of phase 1, then of each phase-2 chunk
   const bool nk = b->op == POYHIP_OP_NEWKK_ALIGN;
+  const int per = nk ? 1 : kLinCounters;
+  const int nzero = per * (n + 2);
+  hipLaunchKernelGGL(k_zero_ints, dim3((nzero + 255) / 256), dim3(256), 0, st, b->d_counters,
+                     nzero);
+  PairTable all = batch_table(b, d_blob, d_off1, d_off2, -1);
   if (!nk)
     hipLaunchKernelGGL(k_linear_deltawh, dim3((n + kDwPairsPerBlock - 1) / kDwPairsPerBlock),
                        dim3(64 * kDwPairsPerBlock), 0, st, all, b->d_dw,
@@ -1712,6 +1828,7 @@ int batch_run_two_phase(poyhip_batch* b, const uint8_t* d_blob, const int64_t* d
   A.res = b->d_res;
   A.counter = b->d_counters;
   A.phase = 1;
+  A.budget = b->dm_budget;
   NkFillArgs N;
   N.pt = all;
   N.cm = c->d_cm;
@@ -1728,7 +1845,7 @@ int batch_run_two_phase(poyhip_batch* b, const uint8_t* d_blob, const int64_t* d
   N.medians = 1;
   HIPCHK(c, hipEventRecord(ev[1], st));
   if (nk) HIPCHK(c, launch_newkk_fill(N, false, b->wide, b->grid, st));
-  else HIPCHK(c, launch_linear_fill(c, A, false, b->grid, st));
+  else HIPCHK(c, launch_linear_fill(c, A, false, b->grid, b->max_sum, true, st));
   HIPCHK(c, hipEventRecord(ev[2], st));
   b->h_res.resize(n);
   HIPCHK(c, hipMemcpyAsync(b->h_res.data(), b->d_res, sizeof(PairResult) * (size_t)n,
@@ -1745,7 +1862,8 @@ int batch_run_two_phase(poyhip_batch* b, const uint8_t* d_blob, const int64_t* d
     const PairResult& r = b->h_res[k];
     const int64_t exact =
         nk ? (r.full == 2 ? 0 : nk_dm_exact(b->la[k], b->lb[k], r.newk))
-           : lin_dm_exact(b->la[k], b->lb[k], r.newk < 0 ? 0 : r.newk, r.full != 0);
+           : lin_region_bytes(b->la[k], b->lb[k], r.newk < 0 ? 0 : r.newk, (r.full & 1) != 0,
+                              b->dm_budget);
     const int64_t sz = (exact + 255) & ~(int64_t)255;
     if (sz > b->dm_budget)
       return set_err(c, POYHIP_ECAP, "pair %d needs %lld direction bytes", k, (long long)sz);
@@ -1763,14 +1881,14 @@ int batch_run_two_phase(poyhip_batch* b, const uint8_t* d_blob, const int64_t* d
   for (size_t k = 0; k < b->chunks.size(); k++) {
     PairTable t = batch_table(b, d_blob, d_off1, d_off2, (int)k);
     A.pt = t;
-    A.counter = b->d_counters + 1 + k;
+    A.counter = b->d_counters + per * (1 + k);
     A.phase = 2;
     N.pt = t;
-    N.counter = b->d_counters + 1 + k;
+    N.counter = b->d_counters + per * (1 + k);
     N.phase = 2;
     HIPCHK(c, hipEventRecord(ev[1], st));
     if (nk) HIPCHK(c, launch_newkk_fill(N, true, b->wide, b->grid, st));
-    else HIPCHK(c, launch_linear_fill(c, A, true, b->grid, st));
+    else HIPCHK(c, launch_linear_fill(c, A, true, b->grid, b->max_sum, true, st));
     HIPCHK(c, hipEventRecord(ev[2], st));
     if (!nk) {
       LinBtArgs B;

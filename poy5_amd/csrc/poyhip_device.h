@@ -140,15 +140,18 @@ __device__ __forceinline__ uint32_t dm_word(const uint8_t* dm, long long cap, bo
 
 // Exclusive prefix sum over the 64 lanes (Hillis-Steele with shuffles) and
 // the total.
-__device__ __forceinline__ int wave_excl_sum(int x, int& total) {
+__device__ __forceinline__ int wave_excl_sum_lane(int x, int lane, int& total) {
   int v = x;
 #pragma unroll
   for (int d = 1; d < 64; d <<= 1) {
     const int y = __shfl_up(v, d);
-    if ((int)threadIdx.x >= d) v += y;
+    if (lane >= d) v += y;
   }
   total = __builtin_amdgcn_readlane(v, 63);
   return v - x;
+}
+__device__ __forceinline__ int wave_excl_sum(int x, int& total) {
+  return wave_excl_sum_lane(x, (int)threadIdx.x, total);
 }
 
 }  // namespace poyhip

@@ -36,6 +36,18 @@ POYHIP_HD inline int64_t lin_ws_ints(int Lb) { return (int64_t)4 * Lb + 16; }
 POYHIP_HD inline int64_t lin_dm_bytes(int La, int Lb) {
   return (int64_t)n_stripes(La) * (((int64_t)Lb + 63 + 15) >> 4) * 256;
 }
+// the diagonal layout of a round with band half-width newk (D = Lb - La):
+// slots of an even and the next odd diagonal from -newk (made even) to
+// D + newk, a word of 16 steps x 2 bits per slot, block after block
+POYHIP_HD inline int diag_slots(int D, int newk) {
+  return (D + newk + ((newk + 1) & ~1)) / 2 + 1;
+}
+POYHIP_HD inline int diag_stride(int D, int newk) { return (diag_slots(D, newk) + 7) & ~7; }
+POYHIP_HD inline int64_t diag_dm_bytes(int La, int Lb, int newk) {
+  const int64_t nblk = ((La + Lb - 2) >> 4) + 1;
+  // whole 256-byte lines, so that a sweep's rounds follow one another
+  return (nblk * diag_stride(Lb - La, newk) * 4 + 255) & ~(int64_t)255;
+}
 // outputs: r1, r2 (La+Lb each), ancestor median (La+Lb+1), median with gaps
 POYHIP_HD inline int64_t lin_out_cap(int La, int Lb) { return (int64_t)La + Lb + 1; }
 POYHIP_HD inline int64_t lin_out_bytes(int La, int Lb) { return 4 * lin_out_cap(La, Lb); }

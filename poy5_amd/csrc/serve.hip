@@ -222,6 +222,7 @@ int srv_launch(poyhip_server* s, SrvSlot& sl) {
   std::vector<double> work(n);
   int64_t dmo = 0, so = 0, oo = 0;
   int nkeep = 0, maxlb = 1;
+  int64_t max_sum = 0;
   for (int k = 0; k < n; k++) {
     SrvRequest* r = sl.reqs[k];
     const PoolEntry& ea = s->entries[r->a];
@@ -241,6 +242,7 @@ int srv_launch(poyhip_server* s, SrvSlot& sl) {
     t.out_off[k] = oo;
     oo += srv_out_bytes(op, t.la[k], t.lb[k]);
     maxlb = std::max(maxlb, t.lb[k]);
+    max_sum = std::max(max_sum, (int64_t)t.la[k] + t.lb[k]);
     work[k] = (double)t.la[k] * t.lb[k];
     if (op == POYHIP_OP_ALIGN_2D && (r->flags & POYHIP_REQ_KEEP_MEDIAN)) {
       t.keep_pid[nkeep] = k;
@@ -294,7 +296,7 @@ int srv_launch(poyhip_server* s, SrvSlot& sl) {
   pt.npairs = n;
   const int grid = std::min(n, s->grid);
   const long long wss = (ws_ints(op, maxlb) + 63) & ~63LL;
-  hipLaunchKernelGGL(k_zero_ints, dim3(1), dim3(64), 0, st, sl.d_counters, 2);
+  hipLaunchKernelGGL(k_zero_ints, dim3(1), dim3(64), 0, st, sl.d_counters, kLinCounters);
   if (op == POYHIP_OP_ALIGN_AFFINE)
     hipLaunchKernelGGL(k_affine_classify, dim3(n), dim3(64), 0, st, pt, sl.d_cls, nullptr);
   if (!op_is_affine(op))
@@ -352,7 +354,7 @@ int srv_launch(poyhip_server* s, SrvSlot& sl) {
     A.counter = sl.d_counters;
     A.phase = 0;
     if (op == POYHIP_OP_ALIGN_2D) {
-      HIPCHK(c, launch_linear_fill(c, A, true, grid, st));
+      HIPCHK(c, launch_linear_fill(c, A, true, grid, max_sum, true, st));
       LinBtArgs B;
       B.pt = pt;
       B.cm = c->d_cm;
@@ -366,7 +368,7 @@ int srv_launch(poyhip_server* s, SrvSlot& sl) {
         hipLaunchKernelGGL(k_pool_store, dim3(nkeep), dim3(64), 0, st, sl.d_out, dt.out_off,
                            dt.keep_cap, sl.d_outlen, dt.keep_pid, dt.keep_pool, s->d_pool, nkeep);
     } else {
-      HIPCHK(c, launch_linear_fill(c, A, false, grid, st));
+      HIPCHK(c, launch_linear_fill(c, A, false, grid, max_sum, true, st));
     }
   }
   hipLaunchKernelGGL(k_extract_cost, dim3((n + 255) / 256), dim3(256), 0, st, sl.d_res, sl.d_cost,
