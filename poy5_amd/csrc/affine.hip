@@ -35,30 +35,12 @@ struct AffFillArgs {
   uint8_t* out = nullptr;
   int* outlen = nullptr;
   int rotating = 1;  // 0: gap-free pairs also run the plain stripe loop
-  // the anti-diagonal fill (affine_diag.hip): bits of a gap count in its
-  // keys, the number of pairs an earlier fill left (their results say
-  // kAffLeft; a fill with left_in takes only those) and left to the next
-  int nd = 0;
-  const int* left_in = nullptr;
-  int* left_out = nullptr;
 };
-
-// PairResult::full of a pair in the anti-diagonal fill's directions, and of
-// one an anti-diagonal fill left
-constexpr int kAffDiag = 2;
-constexpr int kAffLeft = -1;
-
-// direction bytes of a round with band half-width newk in those directions:
-// 8 steps of 4 bits a word, the slots of the linear diagonal layout
-POYHIP_HD inline int64_t aff_diag_bytes(int La, int Lb, int newk) {
-  const int64_t nw = ((La + Lb - 2) >> 4) * 2 + 2;
-  return (nw * diag_stride(Lb - La, newk) * 4 + 255) & ~(int64_t)255;
-}
 
 __device__ __forceinline__ void aff_backtrace_pair(PairTable pt, const uint8_t* dm_all,
                                                    const long long* stab_all, uint8_t* out,
                                                    int* outlen, const uint8_t* s_med, int pid,
-                                                   int newk, bool nib, bool diag, int dm_line);
+                                                   int newk, bool nib);
 
 // The backtrace of pair pid right after its fill, by the same wavefront; the
 // median table goes into s_med (shared memory idle between pairs).
@@ -71,7 +53,7 @@ __device__ __forceinline__ void aff_fused_backtrace(PairTable pt, const CmDev* c
   __threadfence_block();
   for (int k = threadIdx.x; k < 512; k += 64) s_med[k] = cm->median[k];
   __syncthreads();
-  aff_backtrace_pair(pt, dm_all, stab_all, out, outlen, s_med, pid, newk, nib, false, 0);
+  aff_backtrace_pair(pt, dm_all, stab_all, out, outlen, s_med, pid, newk, nib);
   __syncthreads();
 }
 
@@ -695,8 +677,6 @@ __global__ __launch_bounds__(64, 4) void k_affine_fill(AffFillArgs A) {
   const int lane = threadIdx.x;
   // the general kernel has nothing to do when no pair carries a gap bit
   if (!kFast && A.ngen != nullptr && __builtin_amdgcn_readfirstlane(*A.ngen) == 0) return;
-  // nor a stripe fill when the anti-diagonal one left no pair
-  if (A.left_in != nullptr && __builtin_amdgcn_readfirstlane(*A.left_in) == 0) return;
   for (int k = lane; k < kCostN; k += 64)
     s_cost[k] = A.cm->cost[((k >> kRowShift) << 5) + (k & ((1 << kRowShift) - 1))];
   if (lane < 16) s_cost[kCostN + lane] = 0;
@@ -711,7 +691,6 @@ __global__ __launch_bounds__(64, 4) void k_affine_fill(AffFillArgs A) {
     if (q >= A.pt.n) break;
     const int pid = A.pt.order[q];
     if (A.cls != nullptr && A.cls[pid] != (kFast ? 1 : 0)) continue;
-    if (A.left_in != nullptr && A.res[pid].full != kAffLeft) continue;
     const uint8_t* __restrict__ sa = A.pt.blob + rows_off(A.pt, pid);
     const uint8_t* __restrict__ sb = A.pt.blob + cols_off(A.pt, pid);
     const int La = A.pt.len_a[pid], Lb = A.pt.len_b[pid];
@@ -1005,7 +984,7 @@ struct AffBtArgs {
 __device__ __forceinline__ void aff_backtrace_pair(PairTable pt, const uint8_t* dm_all,
                                                    const long long* stab_all, uint8_t* out,
                                                    int* outlen, const uint8_t* s_med, int pid,
-                                                   int newk, bool nib, bool diag, int dm_line) {
+                                                   int newk, bool nib) {
   const int lane = threadIdx.x;
   const uint8_t* sa = pt.blob + rows_off(pt, pid);
   const uint8_t* sb = pt.blob + cols_off(pt, pid);
@@ -1040,78 +1019,6 @@ __device__ __forceinline__ void aff_backtrace_pair(PairTable pt, const uint8_t* 
   int mode = 4;  // 0 vert, 1 horz, 2 diag, 3 align, 4 todo
   int cb = -1, jlo = 0;
   long long base = 0;
-  if (diag) {
-    // anti-diagonal layout: a run of aligned columns stays in one slot's
-    // words, its cells 8 bits apart, so a todo turn takes the aligned columns
-    // down to the next gap of the word (or to the word's start); a gap run
-    // goes on until the cell it reaches says that it opened there
-    const int stride = diag_stride(Lb - La, newk);
-    const int newke = (newk + 1) & ~1;
-    const unsigned* const dw = reinterpret_cast<const unsigned*>(dm) + ((long long)dm_line << 6);
-    int wq = -(1 << 28), wc = 0;  // the window: word rows wq .. wq - 3, slots wc .. wc + 63
-    int nq = -(1 << 28), nc = 0;  // the next one, loading behind it
-    auto word = [&](int q, int c0) __attribute__((always_inline)) -> uint32_t {
-      const int c = c0 + lane;
-      return (q >= 0 && (unsigned)c < (unsigned)stride) ? dw[(long long)q * stride + c] : 0u;
-    };
-    mv = 3;
-    while (i != 0 && j != 0) {
-      const int q = (i + j) >> 3, u = (i + j) & 7;
-      const int c = (j - i + newke) >> 1;
-      if (q > wq || q < wq - 3 || c < wc || c >= wc + 64) {
-        if (q <= nq && q >= nq - 3 && c >= nc && c < nc + 64) {
-          wa0 = wb0; wa1 = wb1; wa2 = wb2; wa3 = wb3;
-          wq = nq;
-          wc = nc;
-        } else {
-          wq = q;
-          wc = c - 32;
-          wa0 = word(q, wc);
-          wa1 = word(q - 1, wc);
-          wa2 = word(q - 2, wc);
-          wa3 = word(q - 3, wc);
-        }
-        nq = wq - 4;
-        nc = c - 32;
-        wb0 = word(nq, nc);
-        wb1 = word(nq - 1, nc);
-        wb2 = word(nq - 2, nc);
-        wb3 = word(nq - 3, nc);
-      }
-      const int k = wq - q;
-      const uint32_t v = k < 2 ? (k == 0 ? wa0 : wa1) : (k == 2 ? wa2 : wa3);
-      const uint32_t w = __builtin_amdgcn_readlane(v, c - wc);
-      int at = u;  // the cell whose gap move is taken
-      if (mode != 4 && ((w >> (4 * u + 2 + mode)) & 1)) mode = 4;  // the run opened here
-      if (mode == 4) {
-        const uint32_t t =
-            w & ((u & 1) ? 0x30303030u : 0x03030303u) & (0xFFFFFFFFu >> (28 - 4 * u));
-        at = t ? (31 - __builtin_clz(t)) >> 2 : -1;
-        int run = t ? (u - at) >> 1 : (u >> 1) + 1;
-        const int m = imin(i, j);
-        if (run >= m) {
-          run = m;
-          at = -1;
-        }
-        i -= run;
-        j -= run;
-        const int n1 = n + run;
-        if ((n ^ n1) >> 6) {  // at most 4 moves: one chunk boundary
-          ri[cap - 1 - ((n1 & ~63) - 64) - lane] = (uint8_t)mv;
-          mv = 3;
-        }
-        n = n1;
-        if (at < 0) continue;
-        const int nb = (int)(w >> (4 * at)) & 3;
-        mode = (nb & 1) ? ((nb == 3 && pt.prio[pid]) ? 1 : 0) : 1;
-      }
-      record(mode);
-      if ((n & 63) == 0) mv = 3;
-      if (mode == 0) i--;
-      else j--;
-      if (((w >> (4 * at)) & 3) == 3) mode = 4;
-    }
-  }
   while (i != 0 && j != 0) {
     const int bb = (i - 1) >> 6;
     if (bb != cb) {
@@ -1237,21 +1144,6 @@ __device__ __forceinline__ void aff_backtrace_pair(PairTable pt, const uint8_t* 
   }
 }
 
-// The backtraces of the pairs the anti-diagonal fill did.
-__global__ __launch_bounds__(64) void k_affine_diag_backtrace(AffBtArgs A) {
-  __shared__ uint8_t s_med[512];
-  const int lane = threadIdx.x;
-  const int pid = __builtin_amdgcn_readfirstlane(A.pt.order[blockIdx.x]);
-  if (A.cls != nullptr && A.cls[pid] != 1) return;
-  const PairResult R = A.res[pid];
-  if (__builtin_amdgcn_readfirstlane(R.full) != kAffDiag) return;
-  for (int k = lane; k < 512; k += 64) s_med[k] = A.cm->median[k];
-  __syncthreads();
-  aff_backtrace_pair(A.pt, A.dm, A.stab, A.out, A.outlen, s_med, pid,
-                     __builtin_amdgcn_readfirstlane(R.newk), false, true,
-                     __builtin_amdgcn_readfirstlane((int)A.stab[A.pt.stab_off[pid]]));
-}
-
 __global__ __launch_bounds__(64) void k_affine_backtrace(AffBtArgs A) {
   // median table rows 0..15 in shared memory
   __shared__ uint8_t s_med[512];
@@ -1262,8 +1154,7 @@ __global__ __launch_bounds__(64) void k_affine_backtrace(AffBtArgs A) {
   for (int k = lane; k < 512; k += 64) s_med[k] = A.cm->median[k];
   __syncthreads();
   const PairResult R = A.res[pid];
-  aff_backtrace_pair(A.pt, A.dm, A.stab, A.out, A.outlen, s_med, pid, R.newk, R.full != 0, false,
-                     0);
+  aff_backtrace_pair(A.pt, A.dm, A.stab, A.out, A.outlen, s_med, pid, R.newk, R.full != 0);
 }
 
 // algn_CAML_cost_affine_3 (src/algn.c:2457) -> algn_fill_plane_3_aff_nobt

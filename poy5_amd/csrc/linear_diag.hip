@@ -189,7 +189,6 @@ __device__ __forceinline__ void dg_cell(const DiagKey& key, bool sw, int up, int
 // steps of the block and of the last cell and column.
 struct DiagEdge {
   int k0;      // j - i of the lane's first slot's even diagonal
-  int k_first = 0;  // the even diagonal its round starts at
   int s0;      // first step of the block
   int s_fin;   // step of the last cell
   int L2;

@@ -26,7 +26,6 @@
 #include "linear.hip"
 #include "linear_mw.hip"
 #include "linear_diag.hip"
-#include "affine_diag.hip"
 #include "medians.hip"
 #include "newkk.hip"
 #include "unions.hip"
@@ -226,7 +225,7 @@ bool valid_seq(const uint8_t* s, int l) {
 struct OneDesc {
   int64_t off1, off2, dm_off, stab_off, out_off;
   int len_a, len_b, swapped, prio, deltawh, order;
-  int counter[10];  // work counters of the launches, zero (kLinCounters)
+  int counter[8];  // work counters of the launches, zero (kLinCounters)
 };
 constexpr size_t kDescBytes = 128;
 static_assert(sizeof(OneDesc) <= kDescBytes, "descriptor block");
@@ -349,10 +348,9 @@ int64_t lin_ws_slot_ints(int Lb) {
   return std::max(lin_ws_ints(Lb), lin_mw_ws_ints(Lb, kLinMwWaves));
 }
 
-// Work counters of one linear fill, or of one affine align fill: queues and
-// left counts of the anti-diagonal fills' passes, the queues of the stripe
-// fill (4) and, affine, of the general fill (7).
-constexpr int kLinCounters = 10;
+// Work counters of one linear fill: its queue and the count of the pairs it
+// left, of the anti-diagonal fills in turn, then the queue of the stripe fill.
+constexpr int kLinCounters = 8;
 
 // The anti-diagonal fill takes a launch whose costs fit its records and
 // whose sums stay below its out-of-band mark.
@@ -413,40 +411,30 @@ hipError_t launch_linear_fill(poyhip_ctx* c, const LinFillArgs& A0, bool dm, int
     A.left_out = cnt + 1;
     A.nd = lin_key_bits(c, max_sum);
     int cap = DiagGeom<8, 16>::kMaxBand;
-    // pairs left so far are counted in cnt[1], then, after another pass, in
-    // cnt[3] and cnt[6]
-    int* left = cnt + 1;
     if (!A.nd) {
       launch_linear_wide(A, dm, wide_grid, st);
     } else if (n <= c->num_cus) {
       launch_linear_key<16>(A, dm, wide_grid, st);
-    } else if (n <= 6 * c->num_cus) {
-      launch_linear_key<4>(A, dm, std::min(n, c->num_cus * 4), st);
-      cap = DiagGeom<8, 4>::kMaxBand;
-    } else {
+    } else if (n > 6 * c->num_cus) {
+      launch_linear_key<1>(A, dm, std::max(1, std::min(n, c->num_cus * c->waves_per_cu)), st);
       cap = DiagGeom<8, 1>::kMaxBand;
-      launch_linear_key<1>(A, dm, std::min(n, c->num_cus * c->waves_per_cu), st);
-      if (max_band > cap) {
-        A.left_in = left;
-        A.left_out = left = cnt + 3;
-        A.counter = cnt + 2;
-        launch_linear_key<4>(A, dm, std::min(n, c->num_cus * 4), st);
-        cap = DiagGeom<8, 4>::kMaxBand;
-      }
+    } else {
+      launch_linear_key<4>(A, dm, std::max(1, std::min(n, c->num_cus * 4)), st);
+      cap = DiagGeom<8, 4>::kMaxBand;
     }
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     if (max_band > cap && cap < DiagGeom<8, 16>::kMaxBand) {
-      A.left_in = left;
-      A.left_out = left = cnt + 6;
-      A.counter = cnt + 8;
+      A.left_in = cnt + 1;
+      A.left_out = cnt + 3;
+      A.counter = cnt + 2;
       launch_linear_wide(A, dm, wide_grid, st);
       e = hipGetLastError();
       if (e != hipSuccess) return e;
       cap = DiagGeom<8, 16>::kMaxBand;
     }
     if (!dm && max_band <= cap) return hipSuccess;
-    A.left_in = left;
+    A.left_in = A.left_out;
     A.left_out = nullptr;
     A.counter = cnt + 4;
   }
@@ -471,79 +459,6 @@ hipError_t launch_linear_fill(poyhip_ctx* c, const LinFillArgs& A0, bool dm, int
     else
       hipLaunchKernelGGL(k_linear_fill<false>, dim3(grid), dim3(64), 0, st, A);
   }
-  return hipGetLastError();
-}
-
-// Bits of a horizontal gap count in the affine anti-diagonal fill's keys, 0
-// when a launch does not fit them: finite sums, shifted, stay below 2^29 and
-// unshifted below half of POY's HIGH_NUM.
-int aff_key_bits(const poyhip_ctx* c, int64_t max_sum, int max_lb) {
-  const int64_t go = c->cm.gap_open;
-  if (!c->aff_rot || c->lin_max < 0 || go < 0 || max_lb > 65535) return 0;
-  int nd = 1;
-  while (((int64_t)1 << nd) <= max_lb + 1) nd++;
-  const int64_t bound = (max_sum + 4) * std::max(c->lin_max, 1) + 4 * go;
-  return bound < ((int64_t)1 << (29 - nd)) && bound < kHigh / 2 ? nd : 0;
-}
-
-template <int NW>
-void launch_affine_diag(const AffFillArgs& A, int grid, hipStream_t st) {
-  hipLaunchKernelGGL((k_affine_diag<NW>), dim3(grid), dim3(64 * NW), 0, st, A);
-}
-
-// Launches the fill (and, with A.out, the backtraces) of the gap-free pairs
-// of an affine align: the anti-diagonal fill with the wavefronts per pair of
-// launch_linear_fill, more for the pairs whose bands need them, then the
-// stripe fill for what those left.  A.counter[0 .. kLinCounters) is zero.
-hipError_t launch_affine_gapfree(poyhip_ctx* c, const AffFillArgs& A0, int grid, int64_t max_sum,
-                                 int max_lb, hipStream_t st) {
-  AffFillArgs A = A0;
-  const int n = A.pt.n;
-  int* const cnt = A.counter;
-  A.nd = aff_key_bits(c, max_sum, max_lb);
-  if (A.nd) {
-    A.left_out = cnt + 1;
-    int* left = cnt + 1;
-    const int slots = (int)std::min<int64_t>(max_sum / 2 + 2, INT_MAX);  // of the widest band
-    int lanes;
-    if (n <= c->num_cus) {
-      launch_affine_diag<16>(A, n, st);
-      lanes = DiagGeom<4, 16>::kLanes;
-    } else if (n <= 6 * c->num_cus) {
-      launch_affine_diag<4>(A, std::min(n, c->num_cus * 4), st);
-      lanes = DiagGeom<4, 4>::kLanes;
-    } else {
-      lanes = DiagGeom<4, 1>::kLanes;
-      launch_affine_diag<1>(A, std::min(n, c->num_cus * c->waves_per_cu), st);
-      if (slots > 4 * lanes) {
-        A.left_in = left;
-        A.left_out = left = cnt + 3;
-        A.counter = cnt + 2;
-        launch_affine_diag<4>(A, std::min(n, c->num_cus * 4), st);
-        lanes = DiagGeom<4, 4>::kLanes;
-      }
-    }
-    if (slots > 4 * lanes && lanes < DiagGeom<4, 16>::kLanes) {
-      A.left_in = left;
-      A.left_out = left = cnt + 6;
-      A.counter = cnt + 8;
-      launch_affine_diag<16>(A, std::min(n, c->num_cus), st);
-    }
-    A.left_in = left;
-    A.left_out = nullptr;
-    A.counter = cnt + 4;
-    AffBtArgs B;
-    B.pt = A.pt;
-    B.cm = A.cm;
-    B.dm = A.dm;
-    B.stab = A.stab;
-    B.res = A.res;
-    B.out = A.out;
-    B.outlen = A.outlen;
-    B.cls = A.cls;
-    hipLaunchKernelGGL(k_affine_diag_backtrace, dim3(n), dim3(64), 0, st, B);
-  }
-  hipLaunchKernelGGL((k_affine_fill<true, true>), dim3(grid), dim3(64), 0, st, A);
   return hipGetLastError();
 }
 
@@ -1150,7 +1065,7 @@ int poyhip_align_affine_3(poyhip_ctx* c, const uint8_t* si, int li, const uint8_
     // the gap-free kernel runs the backtrace after the fill
     A.out = dout;
     A.outlen = doutlen;
-    HIPCHK(c, launch_affine_gapfree(c, A, 1, (int64_t)li + lj, lj, c->stream));
+    hipLaunchKernelGGL((k_affine_fill<true, true>), dim3(1), dim3(64), 0, c->stream, A);
   }
   HIPCHK(c, hipGetLastError());
   const size_t back = kResBytes + outb;
@@ -1401,7 +1316,6 @@ struct poyhip_batch {
   // 16-bit gap counts carried)
   bool wide = false;
   int64_t max_sum = 0;  // largest L1 + L2
-  int max_lb = 1;       // largest L2
   std::vector<PairResult> h_res;
   // graph replay
   bool use_graph = false;
@@ -1414,9 +1328,6 @@ namespace {
 bool op_is_affine(int op) { return op == POYHIP_OP_ALIGN_AFFINE || op == POYHIP_OP_COST_AFFINE; }
 bool op_is_newkk(int op) { return op == POYHIP_OP_NEWKK_ALIGN || op == POYHIP_OP_NEWKK_COST; }
 bool op_is_linear(int op) { return op == POYHIP_OP_ALIGN_2D || op == POYHIP_OP_COST_2D; }
-int op_counters(int op) {
-  return op_is_linear(op) || op == POYHIP_OP_ALIGN_AFFINE ? kLinCounters : 2;
-}
 bool op_has_dm(int op) {
   return op == POYHIP_OP_ALIGN_AFFINE || op == POYHIP_OP_ALIGN_2D || op == POYHIP_OP_NEWKK_ALIGN;
 }
@@ -1521,14 +1432,14 @@ int batch_enqueue(poyhip_batch* b, const uint8_t* blob, const int64_t* off1, con
   hipStream_t st = c->stream;
   const int nch = (int)b->chunks.size();
   if (timing) HIPCHK(c, hipEventRecord(b->ev[2 * nch], st));
-  // counters: a set per chunk for the align fills and the linear ones, then
-  // the number of general-class pairs; else one per chunk
-  const int nzero = op_counters(b->op) * nch + 1;
+  // counters: two per chunk (fast and general fill queues), then the number
+  // of general-class pairs; a linear fill's own set per chunk
+  const int nzero = op_is_linear(b->op) ? kLinCounters * nch : 2 * nch + 1;
   hipLaunchKernelGGL(k_zero_ints, dim3((nzero + 63) / 64), dim3(64), 0, st, b->d_counters, nzero);
   if (b->op == POYHIP_OP_ALIGN_AFFINE) {
     PairTable all = batch_table(b, blob, off1, off2, -1);
     hipLaunchKernelGGL(k_affine_classify, dim3(b->n), dim3(64), 0, st, all, b->d_cls,
-                       b->d_counters + kLinCounters * nch);
+                       b->d_counters + 2 * nch);
   }
   if (op_is_linear(b->op)) {
     PairTable all = batch_table(b, blob, off1, off2, -1);
@@ -1563,12 +1474,12 @@ int batch_enqueue(poyhip_batch* b, const uint8_t* blob, const int64_t* off1, con
           A.stab = b->d_stab;
           A.res = b->d_res;
           A.cls = b->d_cls;
-          A.ngen = b->d_counters + kLinCounters * nch;
+          A.ngen = b->d_counters + 2 * nch;
           A.out = d_out;  // each pair's backtrace follows its fill
           A.outlen = d_outlen;
-          A.counter = b->d_counters + kLinCounters * k;
-          HIPCHK(c, launch_affine_gapfree(c, A, b->grid, b->max_sum, b->max_lb, st));
-          A.counter += 7;
+          A.counter = b->d_counters + 2 * k;
+          hipLaunchKernelGGL((k_affine_fill<true, true>), dim3(b->grid), dim3(64), 0, st, A);
+          A.counter = b->d_counters + 2 * k + 1;
           hipLaunchKernelGGL((k_affine_fill<true, false>), dim3(b->grid), dim3(64), 0, st, A);
         }
         break;
@@ -1621,7 +1532,7 @@ int batch_enqueue(poyhip_batch* b, const uint8_t* blob, const int64_t* off1, con
       B.out = d_out;
       B.outlen = d_outlen;
       B.cls = b->d_cls;
-      B.ngen = b->d_counters + kLinCounters * nch;
+      B.ngen = b->d_counters + 2 * nch;
       hipLaunchKernelGGL(k_affine_backtrace, dim3(t.n), dim3(64), 0, st, B);
     } else if (b->op == POYHIP_OP_ALIGN_2D) {
       LinBtArgs B;
@@ -1688,7 +1599,6 @@ int poyhip_batch_create(poyhip_ctx* c, int op, int n, const int* len1, const int
     }
   }
   b->wide = maxlb >= 65536 || c->nk_wide_always;
-  b->max_lb = maxlb;
   // largest first (LPT order for the persistent kernels)
   b->order.resize(n);
   std::iota(b->order.begin(), b->order.end(), 0);
@@ -1762,7 +1672,7 @@ int poyhip_batch_create(poyhip_ctx* c, int op, int n, const int* len1, const int
   b->d_order = reinterpret_cast<int*>(p); p += 4 * (size_t)n;
   if (ctx_malloc(c, (void**)&b->d_res, sizeof(PairResult) * (size_t)n) != hipSuccess)
     return fail(POYHIP_ENOMEM, "results");
-  const size_t per = op_counters(op);
+  const size_t per = op_is_linear(op) ? kLinCounters : 2;
   const size_t ncounters = b->two_phase ? per * ((size_t)n + 2) : per * b->chunks.size() + 2;
   if (ctx_malloc(c, (void**)&b->d_counters, sizeof(int) * ncounters) != hipSuccess)
     return fail(POYHIP_ENOMEM, "counters");

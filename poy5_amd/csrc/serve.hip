@@ -320,8 +320,8 @@ int srv_launch(poyhip_server* s, SrvSlot& sl) {
     // takes the pairs with gap-bit symbols
     A.out = sl.d_out;
     A.outlen = sl.d_outlen;
-    HIPCHK(c, launch_affine_gapfree(c, A, grid, max_sum, maxlb, st));
-    A.counter = sl.d_counters + 7;
+    hipLaunchKernelGGL((k_affine_fill<true, true>), dim3(grid), dim3(64), 0, st, A);
+    A.counter = sl.d_counters + 1;
     hipLaunchKernelGGL((k_affine_fill<true, false>), dim3(grid), dim3(64), 0, st, A);
     AffBtArgs B;
     B.pt = pt;
