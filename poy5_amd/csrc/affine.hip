@@ -1163,148 +1163,238 @@ struct AffCostArgs {
   PairTable pt;
   const CmDev* cm;
   int* ws;
-  long long ws_stride;
+  long long ws_stride;  // ints a workgroup
   PairResult* res;
   int* counter;
 };
 
-__global__ __launch_bounds__(64) void k_affine_cost_full(AffCostArgs A) {
+// The full plane of one pair on a workgroup of NW wavefronts, scheduled as
+// the workgroup linear fill (linear_mw.hip): 64-row stripes, stripe b on
+// wavefront b mod NW in the fixed 16-step blocks [P b, P b + nblk), one
+// barrier per block, the row between stripes in global memory (one row of
+// int4 (V, CB, H, ED) per wavefront, row 0 as a stripe -1) loaded one block
+// ahead.  P >= kCostLag: column c leaves lane 63 at step c + 63 of its
+// stripe, five blocks after lane 0's, and is loaded a block before its use.
+//
+// What bounds it: VALU issue, about 55 instructions a step.  With one
+// wavefront per pair, lane 0's loads of the row above inside the step loop
+// made every step wait for memory: 2,048 pairs of 300-1,800 symbols took
+// 24 ms, and the longest pairs alone most of it; they take 3.9 ms here.
+constexpr int kCostWaves = 4;
+constexpr int kCostLag = 6;
+// row entries: columns -16 .. lenj + 111 (loads run a block past the end)
+POYHIP_HD inline int64_t affcost_row(int Lb) { return (int64_t)Lb + 128; }
+POYHIP_HD inline int64_t affcost_ws_ints(int Lb) { return kCostWaves * 4 * affcost_row(Lb); }
+
+// A column's constants: horizontal extension and opening, HAS_GAP_OPENING,
+// and symbol (bits 2..5 the table offset of its bases, bit 0 gap bit, bit 1
+// the previous symbol has none).
+struct CostCol {
+  int ext, open, go, sym;
+};
+
+__global__ __launch_bounds__(64 * kCostWaves) void k_affine_cost_mw(AffCostArgs A) {
+  constexpr int NW = kCostWaves;
   __shared__ int s_cost[1024];
   __shared__ int s_prep[32];
-  const int lane = threadIdx.x;
-  for (int k = lane; k < 1024; k += 64) s_cost[k] = A.cm->cost[k];
-  if (lane < 32) s_prep[lane] = A.cm->prepend[lane];
+  __shared__ int4 s_src[NW][2][16];
+  __shared__ int4 s_out[NW][16];
+  __shared__ CostCol s_col[NW][2][80];
+  __shared__ int s_part[NW];
+  __shared__ int s_pair, s_fin;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  for (int k = tid; k < 1024; k += 64 * NW) s_cost[k] = A.cm->cost[k];
+  if (tid < 32) s_prep[tid] = A.cm->prepend[tid];
   __syncthreads();
   const int go = A.cm->gap_open;
+  int4* const ring = reinterpret_cast<int4*>(A.ws + (long long)blockIdx.x * A.ws_stride);
   for (;;) {
-    const int q = wave_grab(A.counter);
+    if (tid == 0) s_pair = atomicAdd(A.counter, 1);
+    __syncthreads();
+    const int q = __builtin_amdgcn_readfirstlane(s_pair);
+    __syncthreads();  // the next grab rewrites s_pair
     if (q >= A.pt.n) break;
-    const int pid = A.pt.order[q];
+    const int pid = __builtin_amdgcn_readfirstlane(A.pt.order[q]);
     const uint8_t* __restrict__ sa = A.pt.blob + rows_off(A.pt, pid);
     const uint8_t* __restrict__ sb = A.pt.blob + cols_off(A.pt, pid);
-    const int La = A.pt.len_a[pid], Lb = A.pt.len_b[pid];
+    const int La = __builtin_amdgcn_readfirstlane(A.pt.len_a[pid]);
+    const int Lb = __builtin_amdgcn_readfirstlane(A.pt.len_b[pid]);
     const int leni = La - 1, lenj = Lb - 1;
-    const int W1 = lenj + 1;
-    int* bnd = A.ws + (long long)blockIdx.x * A.ws_stride;
-    int rc = 0;
-    if (leni == 0) {
-      // row 0 of initialize_matrices_affine_nobt: H = go + prefix sums
+    const int rs = (int)affcost_row(Lb);
+    const int4* const rin = ring + (long long)((w + NW - 1) % NW) * rs + 16;
+    int4* const rout = ring + (long long)w * rs + 16;
+    // row 0 (initialize_matrices_affine_nobt, src/algn.c:1822-1864): H = go
+    // + prefix sums of the prepend costs, into wavefront NW - 1's row
+    {
+      int4* const r0 = ring + (long long)(NW - 1) * rs + 16;
+      const int per = (Lb + 64 * NW - 1) / (64 * NW);
+      const int a0 = tid * per, a1 = imin(a0 + per, Lb);
       int sum = 0;
-      for (int j = 1 + lane; j <= lenj; j += 64) sum += s_prep[sb[j]];
-      for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o);
-      if (lane == 0) {
-        PairResult r{};
-        r.cost = lenj == 0 ? 0 : go + sum;  // min(H, V=go|HIGH, ED, CB) at lenj
-        if (lenj == 0) r.cost = 0;
-        r.newk = -1;
-        r.rounds = 1;
-        A.res[pid] = r;
+      for (int j = a0; j < a1; j++) sum += j > 0 ? s_prep[sb[j]] : 0;
+      int tot;
+      int run = go + wave_excl_sum_lane(sum, lane, tot);
+      if (lane == 0) s_part[w] = tot;
+      __syncthreads();
+      for (int k = 0; k < w; k++) run += s_part[k];
+      for (int j = a0; j < a1; j++) {
+        run += j > 0 ? s_prep[sb[j]] : 0;
+        r0[j] = j == 0 ? make_int4(go, 0, go, kHigh) : make_int4(kHigh, kHigh, run, kHigh);
       }
-      continue;
-    }
-    const int nstripes = (leni + 63) >> 6;
-    for (int b = 0; b < nstripes; b++) {
-      const int i0 = 1 + (b << 6);
-      const int ilast = imin(i0 + 63, leni);
-      const int i = i0 + lane;
-      const bool act = i <= leni;
-      const int nsteps = W1 + (ilast - i0);
-      int ic = 0, ip = 0, si_ge = 0, si_go = 0, si_ng = 0, si_vext = 0;
-      if (act) {
-        ic = sa[i];
-        ip = sa[i - 1];
-        si_ge = s_cost[(ic << 5) + kGap];
-        si_go = has_gap_opening(i, ip, ic, go);
-        si_ng = ic & 15;
-        si_vext = (i > 1 && (ip & kGap) && !(ic & kGap)) ? si_go + si_ge : si_ge;
-      }
-      const int* rb = bnd + ((b & 1) ^ 1) * 4 * W1;
-      int* wb = bnd + (b & 1) * 4 * W1;
-      int dV = kHigh, dCB = kHigh, dH = kHigh, dED = kHigh;
-      int lH = kHigh, lCB = kHigh;
-      int oV = kHigh, oCB = kHigh, oH = kHigh, oED = kHigh;
-      int h0run = go;
-      int jprev = ldc(sb, -lane - 1, Lb);
-      int jc_next = ldc(sb, -lane, Lb);
-      for (int s = 0; s < nsteps; s++) {
-        const int j = s - lane;
-        const int jc = jc_next;
-        jc_next = ldc(sb, j + 1, Lb);
-        int sV = kHigh, sCB = kHigh, sH = kHigh, sED = kHigh;
-        if (lane == 0) {
-          if (b == 0) {
-            // row 0 (initialize_matrices_affine_nobt, src/algn.c:1822-1864)
-            if (j == 0) { sV = go; sCB = 0; sH = go; sED = kHigh; h0run = go; }
-            else { h0run += s_prep[jc]; sV = kHigh; sCB = kHigh; sH = h0run; sED = kHigh; }
-          } else if (j <= lenj) {
-            sV = rb[j]; sCB = rb[W1 + j]; sH = rb[2 * W1 + j]; sED = rb[3 * W1 + j];
-          }
+      if (leni == 0) {
+        // no DP rows: min(H, V, ED, CB) of row 0's last cell
+        tot = 0;
+        for (int k = 0; k < NW; k++) tot += s_part[k];
+        if (tid == 0) {
+          PairResult r{};
+          r.cost = lenj == 0 ? 0 : go + tot;
+          r.newk = -1;
+          r.rounds = 1;
+          A.res[pid] = r;
         }
-        const int uV = wave_shr1(oV, sV);
-        const int uCB = wave_shr1(oCB, sCB);
-        const int uH = wave_shr1(oH, sH);
-        const int uED = wave_shr1(oED, sED);
-        if (act && j >= 0 && j <= lenj) {
-          int H, V, E, C;
-          if (j == 0) {
-            const int r = uV + si_vext;
-            H = kHigh; E = kHigh; V = r; C = kHigh;
-          } else {
-            const int gr = s_prep[jc];
-            const int sj_go = has_gap_opening(j, jprev, jc, go);
-            const int shx = (j == 1) ? gr : (((jprev & kGap) && !(jc & kGap)) ? sj_go + gr : gr);
-            int ext = lH + shx, opn = lCB + sj_go + gr;
-            H = ext < opn ? ext : opn;
-            // algn_CAML_cost_affine_3 carves its state arrays 2*largest ints
-            // apart but fills them with a row offset of largest + 1
-            // (src/algn.c:2488-2491 with algn_fill_plane_3_aff_nobt's
-            // offset, 2006): an even row's start-of-row writes of H[0] and
-            // E[0] overwrite the odd row's V and C at the last column, so
-            // V at (even i, lenj) has only HIGH sources
-            const bool lost = (j == lenj) && ((i & 1) == 0);
-            ext = (lost ? kHigh : uV) + si_vext;
-            opn = (lost ? kHigh : uCB) + si_go + si_ge;
-            V = ext < opn ? ext : opn;
-            const bool flag = (kGap & ic) && (kGap & jc);
-            const bool flag2 = !(kGap & ip) && !(kGap & jprev);
-            const int dg = flag ? 0 : kHigh;
-            const int od = flag ? (flag2 ? 0 : 2 * go) : kHigh;
-            ext = dED + dg; opn = dCB + od;
-            E = ext < opn ? ext : opn;
-            const int d = s_cost[(si_ng << 5) + (jc & 15)];
-            const int extra = (sj_go < si_go) ? si_go : sj_go;
-            // with lenj = 1 the same overlap makes an odd row's own V and
-            // E of column 1 land on the H and V of column 0 of the row
-            // above before the aligned state reads them
-            const bool self1 = (lenj == 1) && ((i & 1) == 1);
-            int cb = dCB + d;
-            const int fv = (self1 ? E : dV) + d + ((ic == si_ng) ? 0 : sj_go);
-            const int fh = (self1 ? V : dH) + d + ((jc == (jc & 15)) ? 0 : si_go);
-            const int fd = dED + d + extra;
-            if (cb > fv) cb = fv;
-            if (cb > fh) cb = fh;
-            if (cb > fd) cb = fd;
-            C = cb;
-          }
-          oV = V; oCB = C; oH = H; oED = E;
-          lH = H; lCB = C;
-          if (i == leni && j == lenj) rc = imin(imin(H, V), imin(E, C));
-          if (lane == 63) { wb[j] = V; wb[W1 + j] = C; wb[2 * W1 + j] = H; wb[3 * W1 + j] = E; }
-        }
-        dV = uV; dCB = uCB; dH = uH; dED = uED;
-        jprev = jc;
+        __syncthreads();
+        continue;
       }
-      __threadfence_block();
     }
-    const int cost = __builtin_amdgcn_readfirstlane(__shfl(rc, (leni - 1) & 63));
-    if (lane == 0) {
+    const int nst = (leni + 63) >> 6;
+    const int nblk = (lenj + 1 + 63 + 15) >> 4;
+    const int P = imax(kCostLag, (nblk + NW - 1) / NW);
+    const int Q = P * (nst - 1) + nblk;
+    __syncthreads();  // row 0 written
+    int b = w;
+    // per-stripe state
+    int i = 0, crow = 0, ge_v = 0, go_r = 0, goge = 0;
+    bool act = false, gap = false, ipng = false, isng = false;
+    int dV = kHigh, dCB = kHigh, dH = kHigh, dED = kHigh, lH = kHigh, lCB = kHigh;
+    int oV = kHigh, oCB = kHigh, oH = kHigh, oED = kHigh;
+    auto col_rec = [&](int j) __attribute__((always_inline)) {
+      CostCol c{0, 0, 0, 0};
+      if ((unsigned)j <= (unsigned)lenj) {
+        const int jc = sb[j], jp = j > 0 ? sb[j - 1] : sb[0];
+        const int gr = s_prep[jc];
+        c.go = has_gap_opening(j, jp, jc, go);
+        c.ext = (j != 1 && (jp & kGap) && !(jc & kGap)) ? c.go + gr : gr;
+        c.open = c.go + gr;
+        c.sym = ((jc & 15) << 2) | ((jc >> 4) & 1) | ((jp & kGap) ? 0 : 2);
+      }
+      return c;
+    };
+    auto enter = [&]() {
+      i = 1 + (b << 6) + lane;
+      act = i <= leni;
+      const int ir = imin(i, leni);
+      const int ic = sa[ir], ip = sa[ir - 1];
+      const int ge = s_cost[(ic << 5) + kGap];
+      go_r = has_gap_opening(ir, ip, ic, go);
+      ge_v = (ir > 1 && (ip & kGap) && !(ic & kGap)) ? go_r + ge : ge;
+      goge = go_r + ge;
+      gap = (ic & kGap) != 0;
+      isng = !gap;
+      ipng = !(ip & kGap);
+      crow = (ic & 15) << 5;
+      dV = dCB = dH = dED = lH = lCB = oV = oCB = oH = oED = kHigh;
+      if (lane < 16) s_src[w][0][lane] = rin[lane];
+      for (int k = lane; k < 80; k += 64) s_col[w][0][k] = col_rec(k - 63);
+    };
+    bool in = false;
+    for (int qb = 0; qb < Q; qb++) {
+      if (!in && b < nst && qb == P * b) {
+        enter();
+        in = true;
+        __builtin_amdgcn_wave_barrier();
+      }
+      if (in) {
+        const int m = qb - P * b, s0 = m << 4, buf = m & 1;
+        const bool more = m + 1 < nblk;
+        int4 nsrc = make_int4(0, 0, 0, 0);
+        CostCol nc0{0, 0, 0, 0}, nc1{0, 0, 0, 0};
+        if (more) {
+          if (lane < 16) nsrc = rin[s0 + 16 + lane];
+          nc0 = col_rec(s0 + 16 - 63 + lane);
+          if (lane < 16) nc1 = col_rec(s0 + 16 + 1 + lane);
+        }
+        const CostCol* const cw = &s_col[w][buf][63 - lane];
+        // every lane past column 0 and before the last one for all 16 steps
+        const bool inner = s0 >= 64 && s0 + 15 <= lenj - 1;
+        auto step = [&](const int u, auto edge_t) __attribute__((always_inline)) {
+          constexpr bool kEdge = decltype(edge_t)::value;
+          const int j = s0 + u - lane;
+          const CostCol c = cw[u];
+          const int4 src = s_src[w][buf][u];
+          const int uV = wave_shr1(oV, src.x);
+          const int uCB = wave_shr1(oCB, src.y);
+          const int uH = wave_shr1(oH, src.z);
+          const int uED = wave_shr1(oED, src.w);
+          const bool jgap = c.sym & 1;
+          int H = imin(lH + c.ext, lCB + c.open);
+          int vx = uV, vo = uCB;
+          // algn_CAML_cost_affine_3 carves its state arrays 2*largest ints
+          // apart but fills them with a row offset of largest + 1
+          // (src/algn.c:2488-2491 with algn_fill_plane_3_aff_nobt's offset,
+          // 2006): an even row's start-of-row writes of H[0] and E[0]
+          // overwrite the odd row's V and C at the last column, so V at
+          // (even i, lenj) has only HIGH sources
+          if (kEdge && j == lenj && (i & 1) == 0) vx = vo = kHigh;
+          int V = imin(vx + ge_v, vo + goge);
+          const bool both = gap && jgap;
+          const int dg = both ? 0 : kHigh;
+          const int od = both ? ((ipng && (c.sym & 2)) ? 0 : 2 * go) : kHigh;
+          int E = imin(dED + dg, dCB + od);
+          const int d = s_cost[crow + ((c.sym >> 2) & 15)];
+          // with lenj = 1 the same overlap makes an odd row's own V and E of
+          // column 1 land on the H and V of column 0 of the row above before
+          // the aligned state reads them
+          const bool self = kEdge && lenj == 1 && (i & 1) == 1;
+          const int fv = (self ? E : dV) + (isng ? 0 : c.go);
+          const int fh = (self ? V : dH) + (jgap ? go_r : 0);
+          const int fd = dED + imax(c.go, go_r);
+          int C = imin(imin(dCB, fv), imin(fh, fd)) + d;
+          if (kEdge && j == 0) {
+            V = uV + ge_v;
+            H = E = C = kHigh;
+          }
+          if (!kEdge || (act && j >= 0 && j <= lenj)) {
+            oV = V; oCB = C; oH = H; oED = E;
+            lH = H; lCB = C;
+          }
+          if (kEdge && i == leni && j == lenj) s_fin = imin(imin(H, V), imin(E, C));
+          if (lane == 63) s_out[w][u] = make_int4(oV, oCB, oH, oED);
+          dV = uV; dCB = uCB; dH = uH; dED = uED;
+        };
+        if (inner) {
+#pragma unroll
+          for (int u = 0; u < 16; u++) step(u, std::false_type{});
+        } else {
+#pragma unroll 2
+          for (int u = 0; u < 16; u++) step(u, std::true_type{});
+        }
+        // lane 63's 16 results to this wavefront's row, the next block's
+        // sources to LDS
+        __builtin_amdgcn_wave_barrier();
+        if (lane < 16) {
+          const int jc = s0 + lane - 63;
+          if (jc >= 0 && jc <= lenj) rout[jc] = s_out[w][lane];
+        }
+        if (more) {
+          if (lane < 16) s_src[w][buf ^ 1][lane] = nsrc;
+          s_col[w][buf ^ 1][lane] = nc0;
+          if (lane < 16) s_col[w][buf ^ 1][64 + lane] = nc1;
+        } else {
+          b += NW;
+          in = false;
+        }
+      }
+      __syncthreads();
+    }
+    if (tid == 0) {
       PairResult r{};
-      r.cost = cost;
+      r.cost = s_fin;
       r.newk = leni - 1;
       r.rounds = 1;
       r.cells = (long long)leni * (lenj + 1);
       A.res[pid] = r;
     }
+    __syncthreads();
   }
 }
 

@@ -1001,7 +1001,7 @@ int poyhip_cost_affine_3(poyhip_ctx* c, const uint8_t* si, int li, const uint8_t
   A.ws_stride = 0;
   A.res = static_cast<PairResult*>(c->outblk.p);
   A.counter = counter;
-  hipLaunchKernelGGL(k_affine_cost_full, dim3(1), dim3(64), 0, c->stream, A);
+  hipLaunchKernelGGL(k_affine_cost_mw, dim3(1), dim3(64 * kCostWaves), 0, c->stream, A);
   HIPCHK(c, hipGetLastError());
   PairResult r;
   HIPCHK(c, hipMemcpyAsync(&r, c->outblk.p, sizeof r, hipMemcpyDeviceToHost, c->stream));
@@ -1461,7 +1461,7 @@ int batch_enqueue(poyhip_batch* b, const uint8_t* blob, const int64_t* off1, con
           A.ws_stride = b->ws_stride;
           A.res = b->d_res;
           A.counter = b->d_counters + k;
-          hipLaunchKernelGGL(k_affine_cost_full, dim3(b->grid), dim3(64), 0, st, A);
+          hipLaunchKernelGGL(k_affine_cost_mw, dim3(b->grid), dim3(64 * kCostWaves), 0, st, A);
         } else {
           // gap-free pairs on the fast kernel, the others on the general one
           AffFillArgs A;
@@ -1649,6 +1649,8 @@ int poyhip_batch_create(poyhip_ctx* c, int op, int n, const int* len1, const int
   for (const auto& ch : b->chunks) b->dm_cap = std::max(b->dm_cap, ch.dm_bytes);
   // persistent grid: waves resident across the device
   b->grid = std::min(n, c->num_cus * c->waves_per_cu);
+  if (op == POYHIP_OP_COST_AFFINE)  // workgroups of kCostWaves
+    b->grid = std::min(n, c->num_cus * std::max(1, c->waves_per_cu / kCostWaves));
   if (b->grid < 1) b->grid = 1;
   b->ws_stride = (ws_ints(op, maxlb) + 63) & ~63LL;
   // device allocations

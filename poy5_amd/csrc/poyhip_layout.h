@@ -26,9 +26,6 @@ POYHIP_HD inline int64_t aff_dm_bytes(int La, int Lb) {
 // outputs: resi, resj, median, medianwg, each La+Lb+2 bytes
 POYHIP_HD inline int64_t aff_out_bytes(int La, int Lb) { return 4 * (int64_t)(La + Lb + 2); }
 
-// ---- full affine cost (no directions) -----------------------------------
-POYHIP_HD inline int64_t affcost_ws_ints(int Lb) { return (int64_t)8 * Lb + 16; }
-
 // ---- non-affine ---------------------------------------------------------
 // per-wavefront workspace: two boundary rows of (cost, delete count)
 POYHIP_HD inline int64_t lin_ws_ints(int Lb) { return (int64_t)4 * Lb + 16; }

@@ -341,7 +341,8 @@ int srv_launch(poyhip_server* s, SrvSlot& sl) {
     A.ws_stride = wss;
     A.res = sl.d_res;
     A.counter = sl.d_counters;
-    hipLaunchKernelGGL(k_affine_cost_full, dim3(grid), dim3(64), 0, st, A);
+    hipLaunchKernelGGL(k_affine_cost_mw, dim3(std::min(grid, c->num_cus * 4)),
+                       dim3(64 * kCostWaves), 0, st, A);
   } else {
     LinFillArgs A;
     A.pt = pt;
@@ -502,7 +503,8 @@ int poyhip_server_create(poyhip_ctx* c, const poyhip_server_opts* o, poyhip_serv
   // outputs of a full slot: capped like the direction stores
   s->slot_out = std::max<int64_t>((int64_t)d.slot_dm_bytes / 8, aff_out_bytes(d.max_len, d.max_len) * 4);
   s->grid = std::min(d.max_batch_pairs, c->num_cus * 8);
-  s->ws_stride = (std::max(aff_ws_ints(d.max_len), lin_ws_slot_ints(d.max_len)) + 63) & ~63LL;
+  s->ws_stride = (std::max({aff_ws_ints(d.max_len), lin_ws_slot_ints(d.max_len),
+                            affcost_ws_ints(d.max_len)}) + 63) & ~63LL;
   auto fail = [&](const char* what) {
     srv_free(s);
     delete s;
