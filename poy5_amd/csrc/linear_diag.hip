@@ -77,11 +77,54 @@ struct DiagRec {
   unsigned off;
   int cost;
 };
+// The wide form holds both in one register (offset below, cost above): its
+// eight slots a lane spill less of their 128 registers than with two (128
+// pairs of 16,000-100,000 symbols: 1.36 s in the stripe fills, 1.16 s with two
+// registers a record, 1.02 s with one).
+struct DiagPacked {
+  unsigned v;
+};
+template <bool kKey>
+struct DiagRecOf {
+  typedef DiagRec type;
+};
+template <>
+struct DiagRecOf<false> {
+  typedef DiagPacked type;
+};
 
-template <int NW>
+__device__ __forceinline__ DiagRec dg_rec(DiagRec*, unsigned off, int cost) {
+  return DiagRec{off, cost};
+}
+__device__ __forceinline__ DiagPacked dg_rec(DiagPacked*, unsigned off, int cost) {
+  return DiagPacked{off | ((unsigned)cost << 16)};
+}
+__device__ __forceinline__ int dg_cost(DiagRec r) { return r.cost; }
+__device__ __forceinline__ int dg_cost(DiagPacked r) { return (int)(r.v >> 16); }
+__device__ __forceinline__ unsigned dg_off(DiagRec r) { return r.off; }
+__device__ __forceinline__ unsigned dg_off(DiagPacked r) { return r.v & 0xFFFFu; }
+// table offset of a row and a column symbol
+__device__ __forceinline__ unsigned dg_addr(DiagRec a, DiagRec b) { return a.off + b.off; }
+__device__ __forceinline__ unsigned dg_addr(DiagPacked a, DiagPacked b) {
+  unsigned r;  // 16-bit adds clear the upper half
+  asm("v_add_u16_e32 %0, %1, %2" : "=v"(r) : "v"(a.v), "v"(b.v));
+  return r;
+}
+// x + the record's cost
+__device__ __forceinline__ int dg_plus(int x, DiagRec r) { return x + r.cost; }
+__device__ __forceinline__ int dg_plus(int x, DiagPacked p) {
+  int r;
+  asm("v_add_u32_sdwa %0, %1, %2 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:WORD_1"
+      : "=v"(r)
+      : "v"(x), "v"(p.v));
+  return r;
+}
+
+template <int NW, bool kKey>
 struct DiagShared {
-  DiagRec row[32];
-  DiagRec col[32];
+  typedef typename DiagRecOf<kKey>::type Rec;
+  Rec row[32];
+  Rec col[32];
   int tab[33 * 64];
   int tail[32];
   int tail_below;  // some tail cost is below its symbol's deletion cost
@@ -93,12 +136,13 @@ struct DiagShared {
   int halo[NW > 1 ? 2 : 1][NW > 1 ? NW : 1][2][NW > 1 ? 32 : 1];
 };
 
-template <int R>
+template <int R, bool kKey>
 struct DiagState {
+  typedef typename DiagRecOf<kKey>::type Rec;
   int vE[R], vO[R], dE[R], dO[R];
   int oob[2 * R];    // kDgInf for slots outside the band (even, odd)
-  DiagRec A[R];      // row records i0 - 1 - r before an E step
-  DiagRec B[R];      // column records j0 + r
+  Rec A[R];          // row records i0 - 1 - r before an E step
+  Rec B[R];          // column records j0 + r
 };
 
 __device__ __forceinline__ int dg_from_left(int v) {   // lane - 1's value
@@ -148,12 +192,12 @@ __device__ __forceinline__ unsigned dg_umin3(unsigned a, unsigned b, unsigned c)
 // align, then delete / insert by the swap flag for the move.  `pack` takes
 // the move: bit 0 up, bit 1 not diagonal, earlier steps lower once the block
 // is done (dg_finish).
-template <bool kKey, bool kDm, bool kDc, bool kSw, bool kEdge>
+template <bool kKey, bool kDm, bool kDc, bool kSw, bool kEdge, class Rec>
 __device__ __forceinline__ void dg_cell(const DiagKey& key, bool sw, int up, int left, int diag,
-                                        int del_c, int ins_c, int sub, int udc, int ldc, int oob,
+                                        Rec del_c, Rec ins_c, int sub, int udc, int ldc, int oob,
                                         bool upd, int& v, int& d, unsigned& pack) {
-  const int del = up + del_c;
-  const int ins = left + ins_c;
+  const int del = dg_plus(up, del_c);
+  const int ins = dg_plus(left, ins_c);
   const int aln = diag + sub;
   if (kKey) {
     const unsigned m = dg_umin3((unsigned)del, (unsigned)ins, (unsigned)aln);
@@ -199,19 +243,20 @@ struct DiagEdge {
 // steps ahead of their cells, so that a lone wavefront does not wait for
 // LDS; the group loop bounds the live registers.
 template <int R, bool kKey, bool kDm, bool kDc, bool kSw, int NW, int kMode>
-__device__ __forceinline__ void dg_block(DiagState<R>& S, const DiagShared<NW>& sh,
+__device__ __forceinline__ void dg_block(DiagState<R, kKey>& S, const DiagShared<NW, kKey>& sh,
                                          const DiagKey& key, bool sw, unsigned long long rx,
                                          unsigned long long cx, const DiagEdge& e,
                                          unsigned pack[R]) {
+  typedef typename DiagRecOf<kKey>::type Rec;
   constexpr int P = R <= 2 ? 4 : 2;
   constexpr int kLook = R >= 4 ? 1 : 4 / R;
   constexpr bool kEdge = kMode != kDgInner;
   const char* const tab = reinterpret_cast<const char*>(sh.tab);
-  DiagRec rr[P], cr[P];
+  Rec rr[P], cr[P];
   unsigned rlo = (unsigned)rx, clo = (unsigned)cx;
   unsigned rhi = (unsigned)(rx >> 32), chi = (unsigned)(cx >> 32);
   // the next P records; the symbols move down by P bytes
-  auto records = [&](DiagRec r_[P], DiagRec c_[P]) __attribute__((always_inline)) {
+  auto records = [&](Rec r_[P], Rec c_[P]) __attribute__((always_inline)) {
 #pragma unroll
     for (int t = 0; t < P; t++) {
       r_[t] = sh.row[(rlo >> (8 * t)) & 255u];
@@ -229,12 +274,12 @@ __device__ __forceinline__ void dg_block(DiagState<R>& S, const DiagShared<NW>& 
 #pragma unroll
     for (int r = 0; r < R; r++) {
       const int ia = (u >> 1) - r, jb = ((u + 1) >> 1) + r;
-      sub[u][r] = dg_lds(tab, (ia >= 0 ? rr[ia >= 0 ? ia : 0] : S.A[ia < 0 ? -ia - 1 : 0]).off +
-                                  (jb < R ? S.B[jb < R ? jb : 0] : cr[jb >= R ? jb - R : 0]).off);
+      sub[u][r] = dg_lds(tab, dg_addr(ia >= 0 ? rr[ia >= 0 ? ia : 0] : S.A[ia < 0 ? -ia - 1 : 0],
+                                      jb < R ? S.B[jb < R ? jb : 0] : cr[jb >= R ? jb - R : 0]));
     }
 #pragma unroll 1
   for (int grp = 0; grp < 8 / P; grp++) {
-    DiagRec RA[R - 1 + P], CB[R + P], rn[P], cn[P];
+    Rec RA[R - 1 + P], CB[R + P], rn[P], cn[P];
 #pragma unroll
     for (int r = 0; r < R - 1; r++) RA[R - 2 - r] = S.A[r];
 #pragma unroll
@@ -251,11 +296,11 @@ __device__ __forceinline__ void dg_block(DiagState<R>& S, const DiagShared<NW>& 
 #pragma unroll
       for (int r = 0; r < R; r++) {
         const int ra = R - 1 + (x >> 1) - r, cb = ((x + 1) >> 1) + r;
-        const unsigned va = ra < R - 1 + P ? RA[ra < R - 1 + P ? ra : 0].off
-                                           : rn[ra >= R - 1 + P ? ra - (R - 1 + P) : 0].off;
-        const unsigned vb = cb < R + P ? CB[cb < R + P ? cb : 0].off
-                                       : cn[cb >= R + P ? cb - (R + P) : 0].off;
-        sub[x][r] = dg_lds(tab, va + vb);
+        const Rec va = ra < R - 1 + P ? RA[ra < R - 1 + P ? ra : 0]
+                                      : rn[ra >= R - 1 + P ? ra - (R - 1 + P) : 0];
+        const Rec vb = cb < R + P ? CB[cb < R + P ? cb : 0]
+                                  : cn[cb >= R + P ? cb - (R + P) : 0];
+        sub[x][r] = dg_lds(tab, dg_addr(va, vb));
       }
       const int s = e.s0 + 2 * P * grp + u;
       const int s_upd = s <= e.s_fin ? s : -1;
@@ -265,22 +310,23 @@ __device__ __forceinline__ void dg_block(DiagState<R>& S, const DiagShared<NW>& 
       const int xd = !kDc ? 0 : (odd ? dg_from_right(S.dE[0]) : dg_from_left(S.dO[R - 1]));
 #pragma unroll
       for (int r = 0; r < R; r++) {
-        const DiagRec ra = RA[R - 1 + (u >> 1) - r], cb = CB[((u + 1) >> 1) + r];
-        int del_c = ra.cost;
+        const Rec ra = RA[R - 1 + (u >> 1) - r], cb = CB[((u + 1) >> 1) + r];
+        Rec del_c = ra;
         bool upd = true;
         if (kEdge) {
           const int k = e.k0 + 2 * r + (odd ? 1 : 0);
           upd = imax(k, -k) < s_upd;
           if (kMode == kDgTail && s + k == 2 * (e.L2 - 1))
-            del_c = imin(del_c, dg_lds(tab, ra.off + 32 * 4));
+            del_c = dg_rec((Rec*)nullptr, dg_off(ra),
+                           imin(dg_cost(ra), dg_lds(tab, dg_off(ra) + 32 * 4)));
         }
         if (!odd)
           dg_cell<kKey, kDm, kDc, kSw, kEdge>(key, sw, S.vO[r], r ? S.vO[r ? r - 1 : 0] : xv, S.vE[r], del_c,
-                                   cb.cost, sub[u][r], S.dO[r], r ? S.dO[r ? r - 1 : 0] : xd,
+                                   cb, sub[u][r], S.dO[r], r ? S.dO[r ? r - 1 : 0] : xd,
                                    S.oob[2 * r], upd, S.vE[r], S.dE[r], pack[r]);
         else
           dg_cell<kKey, kDm, kDc, kSw, kEdge>(key, sw, r < R - 1 ? S.vE[r < R - 1 ? r + 1 : 0] : xv, S.vE[r],
-                                   S.vO[r], del_c, cb.cost, sub[u][r],
+                                   S.vO[r], del_c, cb, sub[u][r],
                                    r < R - 1 ? S.dE[r < R - 1 ? r + 1 : 0] : xd, S.dE[r],
                                    S.oob[2 * r + 1], upd, S.vO[r], S.dO[r], pack[r]);
       }
@@ -333,7 +379,7 @@ __device__ __forceinline__ unsigned long long dg_load8(const uint8_t* __restrict
 // (buffer buf; one barrier).  A slot outside the band keeps its own value
 // (its owner may hold no band lane and write nothing).
 template <int R, int NW, bool kKey>
-__device__ __forceinline__ void dg_exchange(DiagShared<NW>& S, DiagState<R>& st, int buf, int w,
+__device__ __forceinline__ void dg_exchange(DiagShared<NW, kKey>& S, DiagState<R, kKey>& st, int buf, int w,
                                             int lane, bool active) {
   constexpr int H = DiagGeom<R, NW>::H;
   const bool lo = lane >= H && lane < 2 * H, hi = lane >= 64 - 2 * H && lane < 64 - H;
@@ -380,7 +426,7 @@ struct DiagSweep {
 // One sweep of a pair on the workgroup: fills the rounds' last values and
 // delete counts; counts the lane-steps into `slots`.
 template <int R, int NW, bool kKey, bool kDm, bool kDc, bool kSw>
-__device__ __forceinline__ void dg_sweep(DiagShared<NW>& S, const DiagKey& key, const uint8_t* __restrict__ sa,
+__device__ __forceinline__ void dg_sweep(DiagShared<NW, kKey>& S, const DiagKey& key, const uint8_t* __restrict__ sa,
                                          const uint8_t* __restrict__ sb, int L1, int L2,
                                          DiagSweep& sp, bool full, bool sw, unsigned* dm,
                                          long long& slots) {
@@ -434,7 +480,7 @@ __device__ __forceinline__ void dg_sweep(DiagShared<NW>& S, const DiagKey& key, 
     rx[b] = dg_load8(sa, L1, i00 + 8 * b, rows_in(b));
     cx[b] = dg_load8(sb, L2, j00 + R + 8 * b, cols_in(b));
   }
-  DiagState<R> st;
+  DiagState<R, kKey> st;
 #pragma unroll
   for (int r = 0; r < R; r++) {
     const int ia = i00 - 1 - r, jb = j00 + r;
@@ -461,7 +507,7 @@ __device__ __forceinline__ void dg_sweep(DiagShared<NW>& S, const DiagKey& key, 
       if (in && k > 0) c = S.tab[kDgPrepend + (sb[k] & 31)];
       if (in && k < 0) {
         const int a = sa[-k] & 31;
-        c = full ? -(kKey ? S.row[a].cost >> (key.nd + 2) : S.row[a].cost) : -S.tail[a];
+        c = full ? -(kKey ? dg_cost(S.row[a]) >> (key.nd + 2) : dg_cost(S.row[a])) : -S.tail[a];
       }
       f[x] = c;
       tot += c;
@@ -630,7 +676,7 @@ __device__ __forceinline__ long long dg_cells(int L1, int L2, int newk, bool ful
 
 template <int NW, bool kKey, bool kDm, bool kDc>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4))) void k_linear_diag(LinFillArgs A) {
-  __shared__ DiagShared<NW> S;
+  __shared__ DiagShared<NW, kKey> S;
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   // a second fill takes only what the first left
@@ -650,11 +696,12 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4))) vo
       S.tab[mw_ag_row(a) + 32] = tl;
       S.tab[kDgPrepend + a] = A.cm->prepend[a];
       S.tail[a] = tl;
-      S.row[a].off = (unsigned)(mw_ag_row(a) * 4);
-      S.row[a].cost = kKey ? (del << sh) | (3 << key.nd) | 1 : del;
-      S.col[a].off = (unsigned)(a * 4);
+      typedef typename DiagRecOf<kKey>::type Rec;
       const int ins = A.cm->cost[(kGap << 5) + a];
-      S.col[a].cost = kKey ? (ins << sh) | (2 << key.nd) : ins;
+      S.row[a] = dg_rec((Rec*)nullptr, (unsigned)(mw_ag_row(a) * 4),
+                        kKey ? (del << sh) | (3 << key.nd) | 1 : del);
+      S.col[a] = dg_rec((Rec*)nullptr, (unsigned)(a * 4),
+                        kKey ? (ins << sh) | (2 << key.nd) : ins);
     }
     if (tid == 0) S.tail_below = below ? 1 : 0;
   }
