@@ -73,6 +73,27 @@ struct AffRow {
   int cost_row;  // (ic & 15) << 5
 };
 
+// A column's constants: horizontal extension and opening, HAS_GAP_OPENING,
+// and symbol (bits 2..5 the table offset of its bases, bit 0 gap bit, bit 1
+// the previous symbol has none).
+struct AffCol {
+  int ext, open, go, sym;
+};
+
+__device__ __forceinline__ AffCol aff_col(const uint8_t* __restrict__ sb, int lenj, int j, int go,
+                                          const int* s_prep) {
+  AffCol c{0, 0, 0, 0};
+  if ((unsigned)j <= (unsigned)lenj) {
+    const int jc = sb[j], jp = j > 0 ? sb[j - 1] : sb[0];
+    const int gr = s_prep[jc];
+    c.go = has_gap_opening(j, jp, jc, go);
+    c.ext = (j != 1 && (jp & kGap) && !(jc & kGap)) ? c.go + gr : gr;
+    c.open = c.go + gr;
+    c.sym = ((jc & 15) << 2) | ((jc >> 4) & 1) | ((jp & kGap) ? 0 : 2);
+  }
+  return c;
+}
+
 struct AffCell {
   int V, C, H, E, G, f, gmax;
   uint32_t code;
@@ -83,17 +104,14 @@ struct AffCell {
 // 127) and the direction byte.  Branch-free: every tie set is the set of
 // sources equal to the minimum, which is what the reference's sequence of
 // comparisons leaves.
-__device__ __forceinline__ void aff_cell(const AffRow& r, int go, int sw, int j, int jc,
-                                         int jprev, bool at_left, bool at_right,
-                                         const int* s_cost, const int* s_prep, int uV, int uCB,
+__device__ __forceinline__ void aff_cell(const AffRow& r, int go, int sw, int j, const AffCol& c,
+                                         int d, bool at_left, bool at_right, int uV, int uCB,
                                          int uG, int dV, int dCB, int dH, int dED, int dG,
                                          int lH, int lCB, int lG, AffCell& o) {
-  const int gr = s_prep[jc];
-  const int sj_go = has_gap_opening(j, jprev, jc, go);
-  const bool jgap = (jc & kGap) != 0;
-  const int shx = (j == 1) ? gr : (((jprev & kGap) && !jgap) ? sj_go + gr : gr);
+  const int sj_go = c.go;
+  const bool jgap = c.sym & 1;
   // horizontal (FILL_EXTEND_HORIZONTAL)
-  const int extH = lH + shx, opnH = lCB + sj_go + gr;
+  const int extH = lH + c.ext, opnH = lCB + c.open;
   const int H = at_left ? kHigh : imin(extH, opnH);
   const int endH = at_left ? 0 : (extH >= opnH);
   // vertical (FILL_EXTEND_VERTICAL)
@@ -102,13 +120,12 @@ __device__ __forceinline__ void aff_cell(const AffRow& r, int go, int sw, int j,
   const int endV = at_right ? 0 : (extV >= opnV);
   // gap-gap block (FILL_EXTEND_BLOCK_DIAGONAL)
   const bool flag = r.gap && jgap;
-  const int jp_ed = at_left ? jc : jprev;
-  const bool flag2 = r.ip_nogap && !(jp_ed & kGap);
+  // at the band's left edge the reference tests the column's own symbol
+  const bool flag2 = r.ip_nogap && !at_left && (c.sym & 2);
   const int dg = flag ? 0 : kHigh;
   const int od = flag ? (flag2 ? 0 : 2 * go) : kHigh;
   const int extE = dED + dg, opnE = dCB + od;
   // align (FILL_CLOSE_BLOCK_DIAGONAL)
-  const int d = s_cost[r.cost_row + (jc & 15)];
   const int fa = dCB + d;
   const int fv = dV + d + (r.isng ? 0 : sj_go);
   const int fh = dH + d + (jgap ? r.go : 0);
@@ -663,20 +680,17 @@ __device__ void rot_round_fast(RotShared& sh, int total, const uint8_t* __restri
 }
 
 // At most 128 VGPRs: four wavefronts per SIMD (shared memory allows as many)
-template <bool kDm, bool kFast>
 __global__ __launch_bounds__(64, 4) void k_affine_fill(AffFillArgs A) {
   // gap-free pairs only index rows and columns 0..15 of the cost table,
   // kept 16 wide (the wavefront's shared memory stays within a sixteenth
   // of the CU's, for four wavefronts per SIMD), plus 16 padding entries
-  constexpr int kCostN = kFast ? 256 : 1024;
-  constexpr int kRowShift = kFast ? 4 : 5;
+  constexpr int kCostN = 256;
+  constexpr int kRowShift = 4;
   __shared__ int s_cost[kCostN + 16];
   __shared__ int s_ge[32];
   __shared__ int s_prep[32];
   __shared__ RotShared s_rot;
   const int lane = threadIdx.x;
-  // the general kernel has nothing to do when no pair carries a gap bit
-  if (!kFast && A.ngen != nullptr && __builtin_amdgcn_readfirstlane(*A.ngen) == 0) return;
   for (int k = lane; k < kCostN; k += 64)
     s_cost[k] = A.cm->cost[((k >> kRowShift) << 5) + (k & ((1 << kRowShift) - 1))];
   if (lane < 16) s_cost[kCostN + lane] = 0;
@@ -690,7 +704,7 @@ __global__ __launch_bounds__(64, 4) void k_affine_fill(AffFillArgs A) {
     const int q = wave_grab(A.counter);
     if (q >= A.pt.n) break;
     const int pid = A.pt.order[q];
-    if (A.cls != nullptr && A.cls[pid] != (kFast ? 1 : 0)) continue;
+    if (A.cls != nullptr && A.cls[pid] != 1) continue;
     const uint8_t* __restrict__ sa = A.pt.blob + rows_off(A.pt, pid);
     const uint8_t* __restrict__ sb = A.pt.blob + cols_off(A.pt, pid);
     const int La = A.pt.len_a[pid], Lb = A.pt.len_b[pid];
@@ -698,8 +712,7 @@ __global__ __launch_bounds__(64, 4) void k_affine_fill(AffFillArgs A) {
     const int leni = La - 1, lenj = Lb - 1, D = lenj - leni;
     const int W1 = lenj + 1;
     int* ws = A.ws + (long long)blockIdx.x * A.ws_stride;
-    uint8_t* dm = A.dm + (kDm ? A.pt.dm_off[pid] : 0);
-    int* EDA = ws;
+    uint8_t* dm = A.dm + A.pt.dm_off[pid];
     int* bnd = ws + aff_bnd_offset(Lb);
     long long* stab = A.stab + A.pt.stab_off[pid];
 
@@ -729,17 +742,13 @@ __global__ __launch_bounds__(64, 4) void k_affine_fill(AffFillArgs A) {
         r.slots = 0;
         A.res[pid] = r;
       }
-      if constexpr (kDm && kFast) {
-        if (A.out != nullptr)
-          aff_fused_backtrace(A.pt, A.cm, A.dm, A.stab, A.out, A.outlen,
-                              reinterpret_cast<uint8_t*>(s_rot.fV), pid, -1, false);
-      }
+      if (A.out != nullptr)
+        aff_fused_backtrace(A.pt, A.cm, A.dm, A.stab, A.out, A.outlen,
+                            reinterpret_cast<uint8_t*>(s_rot.fV), pid, -1, false);
       continue;
     }
 
-    for (int j = lane; j <= lenj; j += 64) EDA[j] = kHigh;
     int HA0 = go;
-    __threadfence_block();
 
     int T = (D + 1) * delta;
     int rounds = 0, newk = 0, cost = 0, gap_num = 0;
@@ -751,9 +760,8 @@ __global__ __launch_bounds__(64, 4) void k_affine_fill(AffFillArgs A) {
       // change: the last cell's gap count is at least D (every path makes D
       // more horizontal than vertical moves, and the count keeps the most
       // horizontal moves over tied paths, exact below 2^16 columns), so
-      // gap_num < p needs p > D.  Gap-free pairs only: the general kernel's
-      // rounds also leave its row-0 gap-gap buffer behind.
-      if constexpr (kFast) {
+      // gap_num < p needs p > D.
+      {
         const int newp = (2 * T - D) / 2;
         if (D >= p && newp - lenj + 1 < 0 && lenj <= 65535) {
           rounds++;
@@ -766,7 +774,7 @@ __global__ __launch_bounds__(64, 4) void k_affine_fill(AffFillArgs A) {
       long long dmpos = 0;
       int rc = 0, rgn = 0;
       int rot_total = -1;
-      if constexpr (kFast && kDm) {
+      {
         int lag = 0;
         if (A.rotating)
           rot_total =
@@ -805,7 +813,7 @@ __global__ __launch_bounds__(64, 4) void k_affine_fill(AffFillArgs A) {
         const int nsteps = (jhi - jlo + 1) + (ilast - i0);
         const int nsteps4 = (nsteps + 3) & ~3;
         // stripe start in steps (gap-free pairs: 32 direction bytes a step)
-        if (kDm && lane == 0) stab[b] = dmpos >> (kFast ? 5 : 6);
+        if (lane == 0) stab[b] = dmpos >> 5;
         slots += (long long)nsteps * 64;
 
         // row constants of lane t (row i); rows past leni get the last row's
@@ -830,18 +838,18 @@ __global__ __launch_bounds__(64, 4) void k_affine_fill(AffFillArgs A) {
         // Up-left cell of lane 0's first step: row i0-1 at column jlo-1.
         // Lane-0 sources are functions of lane 0's column jlo+s only, so the
         // whole wavefront evaluates them with uniform addresses.
-        int dV = kHigh, dCB = kHigh, dH = kHigh, dED = kHigh, dG = 0;
+        int dV = kHigh, dCB = kHigh, dH = kHigh, dG = 0;
         if (jlo >= 1) {
           if (b == 0) {
-            dCB = 0; dH = HA0; dED = EDA[0];
+            dCB = 0; dH = HA0;
           } else {
             const int4 v = rb4[2 * (jlo - 1)];
-            dV = v.x; dCB = v.y; dH = v.z; dED = v.w;
+            dV = v.x; dCB = v.y; dH = v.z;
             dG = reinterpret_cast<const int*>(rb4)[8 * (jlo - 1) + 4];
           }
         }
         int lH = kHigh, lCB = kHigh, lG = 0;
-        int oV = kHigh, oCB = kHigh, oH = kHigh, oED = kHigh, oG = 0;
+        int oV = kHigh, oCB = kHigh, oH = kHigh, oG = 0;
         int cb0run = 0;                               // row-0 prefix at lane 0's column
         int c0prev = sb[imax(jlo - 1, 0)];            // lane 0's previous column symbol
         int jprev = sb[imax(jlo - lane - 1, 0)];      // own previous column symbol
@@ -852,7 +860,7 @@ __global__ __launch_bounds__(64, 4) void k_affine_fill(AffFillArgs A) {
             const int jl0 = jlo + s + u;              // lane 0's column (uniform)
             const int jcl = imin(jl0, lenj);
             const int c0 = sb[jcl];
-            int sV = kHigh, sCB, sH, sED, sG;
+            int sV = kHigh, sCB, sH, sG;
             if (b == 0) {
               // POY's row 0 (algn_newkk_test_aff, src/algn.c:2228-2247)
               const int gr0 = s_prep[c0];
@@ -861,11 +869,10 @@ __global__ __launch_bounds__(64, 4) void k_affine_fill(AffFillArgs A) {
               cb0run = (jl0 == 0) ? 0 : cb0run + add0;
               sCB = cb0run;
               sH = (jl0 == 0) ? HA0 : cb0run;
-              sED = kFast ? kHigh : EDA[jcl];
               sG = jl0 & 0xFFFF;
             } else {
               const int4 v = rb4[2 * jcl];
-              sV = v.x; sCB = v.y; sH = v.z; sED = v.w;
+              sV = v.x; sCB = v.y; sH = v.z;
               sG = reinterpret_cast<const int*>(rb4)[8 * jcl + 4];
             }
             c0prev = c0;
@@ -873,44 +880,28 @@ __global__ __launch_bounds__(64, 4) void k_affine_fill(AffFillArgs A) {
             const int uV = wave_shr1(oV, sV);
             const int uCB = wave_shr1(oCB, sCB);
             const int uH = wave_shr1(oH, sH);
-            const int uED = kFast ? kHigh : wave_shr1(oED, sED);
             const int uG = wave_shr1(oG, sG);
             const int j = jl0 - lane;
             AffCell o;
-            if constexpr (kFast)
-              aff_cell_fast(row, go, sw, j, jc, j == my_lo, j == my_rb, s_cost, s_prep, uV, uCB, uG,
-                            dV, dCB, dH, dG, lH, lCB, lG, o);
-            else
-              aff_cell(row, go, sw, j, jc, jprev, j == my_lo, j == my_rb, s_cost, s_prep, uV, uCB,
-                       uG, dV, dCB, dH, dED, dG, lH, lCB, lG, o);
+            aff_cell_fast(row, go, sw, j, jc, j == my_lo, j == my_rb, s_cost, s_prep, uV, uCB, uG,
+                          dV, dCB, dH, dG, lH, lCB, lG, o);
             const bool inb = j >= my_lo && j <= my_hi;
             if (inb) {
               if (i == leni && j == lenj) { rc = o.f; rgn = o.gmax; }
-              // row-0 buffer persistence across rounds: the last even row of
-              // this round that covers column j leaves its ED value there.
-              if (!kFast && !(i & 1) && i + 2 > imin(leni, j + newk)) EDA[j] = o.E;
               if (lane == 63) {
                 reinterpret_cast<int4*>(wb)[2 * j] = make_int4(o.V, o.C, o.H, o.E);
                 wb[8 * j + 4] = o.G;
               }
             }
-            oV = o.V; oCB = o.C; oH = o.H; oED = o.E; oG = o.G;
+            oV = o.V; oCB = o.C; oH = o.H; oG = o.G;
             lH = o.H; lCB = o.C; lG = o.G;
-            dV = uV; dCB = uCB; dH = uH; dED = uED; dG = uG;
+            dV = uV; dCB = uCB; dH = uH; dG = uG;
             jprev = jc;
-            if constexpr (kFast)
-              pack = (pack << 4) | o.code;  // nibbles, step 0 highest
-            else
-              pack |= o.code << (8 * u);
+            pack = (pack << 4) | o.code;  // nibbles, step 0 highest
           }
-          if constexpr (kDm) {
-            if constexpr (kFast)
-              reinterpret_cast<uint16_t*>(dm + dmpos)[((s >> 2) << 6) + lane] = (uint16_t)pack;
-            else
-              reinterpret_cast<uint32_t*>(dm + dmpos)[((s >> 2) << 6) + lane] = pack;
-          }
+          reinterpret_cast<uint16_t*>(dm + dmpos)[((s >> 2) << 6) + lane] = (uint16_t)pack;
         }
-        dmpos += (long long)(nsteps4 >> 2) * (kFast ? 128 : 256);
+        dmpos += (long long)(nsteps4 >> 2) * 128;
         __threadfence_block();
       }
       const int src = (leni - 1) & 63;
@@ -930,18 +921,354 @@ __global__ __launch_bounds__(64, 4) void k_affine_fill(AffFillArgs A) {
       r.gap_num = gap_num;
       r.newk = newk;
       r.rounds = rounds;
-      r.full = kFast ? 1 : 0;  // direction format: 1 = gap-free nibbles
+      r.full = 1;  // direction format: gap-free nibbles
       r.pad = 0;
       r.cells = cells;
       r.slots = slots;
       A.res[pid] = r;
     }
-    if constexpr (kDm && kFast) {
-      // its median table in the rotating schedule's FIFO
-      if (A.out != nullptr)
-        aff_fused_backtrace(A.pt, A.cm, A.dm, A.stab, A.out, A.outlen,
-                            reinterpret_cast<uint8_t*>(s_rot.fV), pid, newk, kFast);
+    // its median table in the rotating schedule's FIFO
+    if (A.out != nullptr)
+      aff_fused_backtrace(A.pt, A.cm, A.dm, A.stab, A.out, A.outlen,
+                          reinterpret_cast<uint8_t*>(s_rot.fV), pid, newk, true);
+  }
+}
+
+// Pairs with gap-bit symbols: a pair on a workgroup of NW wavefronts.
+// Stripe b of a round runs on wavefront b mod NW in the fixed 16-step blocks
+// [P b, P b + its blocks), one barrier per block; the row between stripes is
+// in global memory (two rows of 8 ints a column: a row is written again two
+// stripes later) and loaded one block ahead, the columns' constants come
+// from LDS.  P >= kGenLag: a stripe starts up to 64 columns right of the one
+// above it, its lane 0's column leaves lane 63 of that stripe up to 127 steps
+// later, and is loaded a block before its use.  Rounds follow each other
+// (each leaves its row-0 gap-gap buffer to the next).
+//
+// What bounds it: the chain of steps of the longest pairs, about 80 (inside
+// the band) to 100 instructions each; a narrow round advances 64 rows in
+// kGenLag blocks however many wavefronts there are.  Loads inside the step
+// loop of one wavefront per pair made every step wait for memory before:
+// 2,048 pairs of 200-2,000 symbols took 33 ms and take 18.4 here, 256 of
+// 3,000 symbols 25.9 and 11.1.
+constexpr int kGenLag = 10;
+
+template <int NW>
+__global__ __launch_bounds__(64 * NW, 4) void k_affine_fill_gen(AffFillArgs A) {
+  __shared__ int s_cost[1024];
+  __shared__ int s_prep[32];
+  __shared__ int4 s_src[NW][2][16];
+  __shared__ int s_srcg[NW][2][16];
+  __shared__ int4 s_out[NW][16];
+  __shared__ int s_outg[NW][16];
+  __shared__ AffCol s_col[NW][2][80];
+  __shared__ int s_part[NW];
+  __shared__ long long s_cells[NW];
+  __shared__ int s_pair, s_fin[2];
+  // nothing to do when no pair carries a gap bit
+  if (A.ngen != nullptr && __builtin_amdgcn_readfirstlane(*A.ngen) == 0) return;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  for (int k = tid; k < 1024; k += 64 * NW) s_cost[k] = A.cm->cost[k];
+  if (tid < 32) s_prep[tid] = A.cm->prepend[tid];
+  __syncthreads();
+  const int go = A.cm->gap_open;
+  const int delta = A.cm->delta;
+  int* const EDA = A.ws + (long long)blockIdx.x * A.ws_stride;
+
+  for (;;) {
+    if (tid == 0) s_pair = atomicAdd(A.counter, 1);
+    __syncthreads();
+    const int q = __builtin_amdgcn_readfirstlane(s_pair);
+    __syncthreads();  // the next grab rewrites s_pair
+    if (q >= A.pt.n) break;
+    const int pid = __builtin_amdgcn_readfirstlane(A.pt.order[q]);
+    if (A.cls != nullptr && __builtin_amdgcn_readfirstlane(A.cls[pid]) != 0) continue;
+    const uint8_t* __restrict__ sa = A.pt.blob + rows_off(A.pt, pid);
+    const uint8_t* __restrict__ sb = A.pt.blob + cols_off(A.pt, pid);
+    const int La = __builtin_amdgcn_readfirstlane(A.pt.len_a[pid]);
+    const int Lb = __builtin_amdgcn_readfirstlane(A.pt.len_b[pid]);
+    const int sw = __builtin_amdgcn_readfirstlane(A.pt.prio[pid]);
+    const int leni = La - 1, lenj = Lb - 1, D = lenj - leni;
+    const int W1 = lenj + 1;
+    uint8_t* const dm = A.dm + A.pt.dm_off[pid];
+    int* const bnd = EDA + aff_bnd_offset(Lb);
+    long long* const stab = A.stab + A.pt.stab_off[pid];
+
+    if (leni == 0) {
+      // No DP rows: the cost is final_cost_matrix[lenj] as set by
+      // initialize_matrices_affine (src/algn.c:1866-1900).
+      int sum = 0;
+      for (int j = 1 + tid; j <= lenj; j += 64 * NW) sum += s_prep[sb[j]];
+      for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o);
+      if (lane == 0) s_part[w] = sum;
+      __syncthreads();
+      int T = (D + 1) * delta, rounds = 0;
+      for (;;) {
+        const int p = (T - D) / 2;
+        rounds++;
+        const int newp = (2 * T - D) / 2;
+        if (65535 < p || newp - lenj + 1 >= 0) break;
+        T *= 2;
+      }
+      if (tid == 0) {
+        sum = 0;
+        for (int k = 0; k < NW; k++) sum += s_part[k];
+        PairResult r{};
+        r.cost = lenj == 0 ? 0 : go + sum;
+        r.gap_num = 65535;
+        r.newk = -1;
+        r.rounds = rounds;
+        A.res[pid] = r;
+      }
+      __syncthreads();
+      continue;
     }
+
+    for (int j = tid; j <= lenj; j += 64 * NW) EDA[j] = kHigh;
+    int HA0 = go;
+    int T = (D + 1) * delta;
+    int rounds = 0, newk = 0, cost = 0, gap_num = 0;
+    long long cells = 0, slots = 0;
+    const int nst = (leni + 63) >> 6;
+    for (;;) {
+      const int p = (T - D) / 2;
+      newk = p >= leni ? leni - 1 : p;
+      auto first_col = [&](int b) { return imax(1 + (b << 6) - newk, 0); };
+      auto n_steps = [&](int b) {
+        const int i0 = 1 + (b << 6), ilast = imin(i0 + 63, leni);
+        const int jhi = ilast + D + newk <= lenj - 1 ? ilast + D + newk : lenj;
+        return (jhi - first_col(b) + 1) + (ilast - i0);
+      };
+      __syncthreads();  // EDA and the row between stripes are free
+      // POY's row 0 (algn_newkk_test_aff, src/algn.c:2228-2247) as the row
+      // above stripe 0, up to its last column
+      {
+        int4* const r0 = reinterpret_cast<int4*>(bnd + 8 * W1);
+        const int n0 = imin(imin(64, leni) + D + newk, lenj) + 1;
+        const int per = (n0 + 64 * NW - 1) / (64 * NW);
+        const int a0 = imin(tid * per, n0), a1 = imin(a0 + per, n0);
+        auto add = [&](int j) __attribute__((always_inline)) {
+          if (j == 0) return 0;
+          const int c = sb[j], cp = sb[j - 1];
+          const int gr = s_prep[c];
+          return ((cp & kGap) && !(c & kGap)) ? has_gap_opening(j, cp, c, go) + gr : gr;
+        };
+        int sum = 0;
+        for (int j = a0; j < a1; j++) sum += add(j);
+        int tot;
+        int run = wave_excl_sum_lane(sum, lane, tot);
+        if (lane == 0) s_part[w] = tot;
+        __syncthreads();
+        for (int k = 0; k < w; k++) run += s_part[k];
+        for (int j = a0; j < a1; j++) {
+          run += add(j);
+          r0[2 * j] = make_int4(kHigh, run, j == 0 ? HA0 : run, EDA[j]);
+          reinterpret_cast<int*>(r0)[8 * j + 4] = j & 0xFFFF;
+        }
+        // stripe starts in steps of 64 bytes
+        if (w == 0) {
+          long long at = 0;
+          for (int b0 = 0; b0 < nst; b0 += 64) {
+            const int b = b0 + lane;
+            const int ns = b < nst ? n_steps(b) : 0;
+            int t4;
+            const int ex = wave_excl_sum_lane((ns + 3) & ~3, lane, t4);
+            if (b < nst) stab[b] = at + ex;
+            at += t4;
+            slots += (long long)ns * 64;
+          }
+        }
+      }
+      // the widest stripe's blocks bound every stripe's
+      const int wide = imin(lenj + 1, 64 + D + 2 * newk) + 63;
+      const int P = imax(kGenLag, (((wide + 15) >> 4) + NW - 1) / NW);
+      const int Q = P * (nst - 1) + ((n_steps(nst - 1) + 15) >> 4);
+      int Qall = Q;  // the last stripes may end in any order
+      for (int b = imax(0, nst - NW); b < nst - 1; b++)
+        Qall = imax(Qall, P * b + ((n_steps(b) + 15) >> 4));
+      __syncthreads();  // row 0 and the stripe table written
+      int b = w;
+      AffRow row{};
+      int i = 0, my_lo = 0, my_rb = 0, jlo = 0, ns = 0, nblk = 0, j_fin = -1;
+      int rc = 0, rgn = 0;
+      unsigned n_ed = 0;
+      long long dmat = 0;
+      int dV = kHigh, dCB = kHigh, dH = kHigh, dED = kHigh, dG = 0;
+      int oV = kHigh, oCB = kHigh, oH = kHigh, oED = kHigh, oG = 0;
+      bool in = false;
+      for (int qb = 0; qb < Qall; qb++) {
+        if (!in && b < nst && qb == P * b) {
+          // enter stripe b: row constants of lane t (row i); rows past leni
+          // get the last row's values and an empty band
+          in = true;
+          const int i0 = 1 + (b << 6);
+          i = i0 + lane;
+          const bool act = i <= leni;
+          jlo = first_col(b);
+          ns = __builtin_amdgcn_readfirstlane(n_steps(b));
+          nblk = (ns + 15) >> 4;
+          dmat = stab[b] << 6;
+          const int ir = imin(i, leni);
+          const int ic = sa[ir], ip = sa[ir - 1];
+          row.gap = ic & kGap;
+          row.isng = (ic & kGap) == 0;
+          row.ip_nogap = (ip & kGap) == 0;
+          row.ge = s_cost[(ic << 5) + kGap];
+          row.go = has_gap_opening(ir, ip, ic, go);
+          row.vext = (ir > 1 && (ip & kGap) && !(ic & kGap)) ? row.go + row.ge : row.ge;
+          row.cost_row = (ic & 15) << 5;
+          my_lo = act ? imax(i - newk, 0) : (1 << 30);
+          my_rb = i + D + newk;
+          const int my_hi = act ? ((my_rb <= lenj - 1) ? my_rb : lenj) : -1;
+          if (act) cells += my_hi - my_lo + 1;
+          j_fin = i == leni ? lenj : -1;
+          // row-0 buffer persistence across rounds: the last even row of this
+          // round that covers column j, i + 2 > min(leni, j + newk), leaves
+          // its ED value there
+          n_ed = 0;
+          if (act && !(i & 1))
+            n_ed = (i + 2 > leni ? my_hi + 1 : imin(my_hi + 1, imax(my_lo, i + 2 - newk))) - my_lo;
+          const int4* const rin = reinterpret_cast<const int4*>(bnd + ((b & 1) ^ 1) * 8 * W1);
+          // up-left cell of lane 0's first step: row i0 - 1, column jlo - 1
+          dV = dCB = dH = dED = kHigh;
+          dG = 0;
+          if (jlo >= 1) {
+            const int4 v = rin[2 * (jlo - 1)];
+            dV = v.x; dCB = v.y; dH = v.z; dED = v.w;
+            dG = reinterpret_cast<const int*>(rin)[8 * (jlo - 1) + 4];
+          }
+          oV = oCB = oH = oED = kHigh;
+          oG = 0;
+          if (lane < 16) {
+            const int jc = imin(jlo + lane, lenj);
+            s_src[w][0][lane] = rin[2 * jc];
+            s_srcg[w][0][lane] = reinterpret_cast<const int*>(rin)[8 * jc + 4];
+          }
+          for (int k = lane; k < 80; k += 64)
+            s_col[w][0][k] = aff_col(sb, lenj, jlo + k - 63, go, s_prep);
+          __builtin_amdgcn_wave_barrier();
+        }
+        if (in) {
+          const int m = qb - P * b, s0 = m << 4, buf = m & 1;
+          const bool more = m + 1 < nblk;
+          int4 nsrc = make_int4(0, 0, 0, 0);
+          int nsg = 0;
+          AffCol nc0{0, 0, 0, 0}, nc1{0, 0, 0, 0};
+          if (more) {
+            const int4* const rin = reinterpret_cast<const int4*>(bnd + ((b & 1) ^ 1) * 8 * W1);
+            if (lane < 16) {
+              const int jc = imin(jlo + s0 + 16 + lane, lenj);
+              nsrc = rin[2 * jc];
+              nsg = reinterpret_cast<const int*>(rin)[8 * jc + 4];
+            }
+            nc0 = aff_col(sb, lenj, jlo + s0 + 16 - 63 + lane, go, s_prep);
+            if (lane < 16) nc1 = aff_col(sb, lenj, jlo + s0 + 17 + lane, go, s_prep);
+          }
+          const AffCol* const cw = &s_col[w][buf][63 - lane];
+          // every lane two columns or more inside its band for all 16 steps,
+          // and none on the last two rows
+          const int i0 = 1 + (b << 6);
+          const bool inner = s0 >= 128 && i0 + 65 <= leni && jlo + s0 + 15 <= lenj &&
+                             jlo + s0 + 15 < i0 + D + newk;
+          uint32_t* const dmw = reinterpret_cast<uint32_t*>(dm + dmat) + (s0 << 4) + lane;
+          auto four = [&](const int t, auto edge_t) __attribute__((always_inline)) {
+            constexpr bool kEdge = decltype(edge_t)::value;
+            uint32_t pack = 0;
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+              const int u = 4 * t + v;
+              const int j = kEdge ? jlo + s0 + u - lane : 1;
+              const AffCol c = cw[u];
+              const int4 src = s_src[w][buf][u];
+              const int uV = wave_shr1(oV, src.x);
+              const int uCB = wave_shr1(oCB, src.y);
+              const int uH = wave_shr1(oH, src.z);
+              const int uED = wave_shr1(oED, src.w);
+              const int uG = wave_shr1(oG, s_srcg[w][buf][u]);
+              AffCell o;
+              aff_cell(row, go, sw, j, c, s_cost[row.cost_row + ((c.sym >> 2) & 15)],
+                       kEdge && j == my_lo, kEdge && j == my_rb, uV, uCB, uG, dV, dCB, dH, dED,
+                       dG, oH, oCB, oG, o);
+              if (kEdge) {
+                rc = j == j_fin ? o.f : rc;
+                rgn = j == j_fin ? o.gmax : rgn;
+                if ((unsigned)(j - my_lo) < n_ed) EDA[j] = o.E;
+              }
+              if (lane == 63) {
+                s_out[w][u] = make_int4(o.V, o.C, o.H, o.E);
+                s_outg[w][u] = o.G;
+              }
+              oV = o.V; oCB = o.C; oH = o.H; oED = o.E; oG = o.G;
+              dV = uV; dCB = uCB; dH = uH; dED = uED; dG = uG;
+              pack |= o.code << (8 * v);
+            }
+            // a stripe's words cover its steps rounded up to four
+            if (s0 + 4 * t < ns) dmw[t << 6] = pack;
+          };
+          if (inner) {
+#pragma unroll 1
+            for (int t = 0; t < 4; t++) four(t, std::false_type{});
+          } else {
+#pragma unroll 1
+            for (int t = 0; t < 4; t++) four(t, std::true_type{});
+          }
+          // lane 63's 16 results (row i0 + 63, inside its band) to the row
+          // between stripes, the next block's sources to LDS
+          __builtin_amdgcn_wave_barrier();
+          if (lane < 16 && i0 + 63 <= leni) {
+            const int jc = jlo + s0 + lane - 63;
+            const int lo = imax(i0 + 63 - newk, 0), rb = i0 + 63 + D + newk;
+            if (jc >= lo && jc <= (rb <= lenj - 1 ? rb : lenj)) {
+              int* const wb = bnd + (b & 1) * 8 * W1;
+              reinterpret_cast<int4*>(wb)[2 * jc] = s_out[w][lane];
+              wb[8 * jc + 4] = s_outg[w][lane];
+            }
+          }
+          if (more) {
+            if (lane < 16) {
+              s_src[w][buf ^ 1][lane] = nsrc;
+              s_srcg[w][buf ^ 1][lane] = nsg;
+            }
+            s_col[w][buf ^ 1][lane] = nc0;
+            if (lane < 16) s_col[w][buf ^ 1][64 + lane] = nc1;
+          } else {
+            if (i == leni) {
+              s_fin[0] = rc;
+              s_fin[1] = rgn;
+            }
+            b += NW;
+            in = false;
+          }
+        }
+        __syncthreads();
+      }
+      cost = __builtin_amdgcn_readfirstlane(s_fin[0]);
+      gap_num = __builtin_amdgcn_readfirstlane(s_fin[1]);
+      rounds++;
+      const int newp = (2 * T - D) / 2;
+      if (gap_num < p || newp - lenj + 1 >= 0) break;
+      if (imin(leni, newk) >= 2) HA0 = kHigh;
+      T *= 2;
+    }
+    for (int o = 32; o > 0; o >>= 1) cells += __shfl_xor(cells, o);
+    if (lane == 0) s_cells[w] = cells;
+    __syncthreads();
+    // wavefront 0's lanes hold the stripe tables' step counts
+    if (w == 0)
+      for (int o = 32; o > 0; o >>= 1) slots += __shfl_xor(slots, o);
+    if (tid == 0) {
+      PairResult r{};
+      r.cost = cost;
+      r.gap_num = gap_num;
+      r.newk = newk;
+      r.rounds = rounds;
+      r.full = 0;  // direction format: bytes
+      r.cells = 0;
+      for (int k = 0; k < NW; k++) r.cells += s_cells[k];
+      r.slots = slots;
+      A.res[pid] = r;
+    }
+    __syncthreads();
   }
 }
 
@@ -1186,20 +1513,13 @@ constexpr int kCostLag = 6;
 POYHIP_HD inline int64_t affcost_row(int Lb) { return (int64_t)Lb + 128; }
 POYHIP_HD inline int64_t affcost_ws_ints(int Lb) { return kCostWaves * 4 * affcost_row(Lb); }
 
-// A column's constants: horizontal extension and opening, HAS_GAP_OPENING,
-// and symbol (bits 2..5 the table offset of its bases, bit 0 gap bit, bit 1
-// the previous symbol has none).
-struct CostCol {
-  int ext, open, go, sym;
-};
-
 __global__ __launch_bounds__(64 * kCostWaves) void k_affine_cost_mw(AffCostArgs A) {
   constexpr int NW = kCostWaves;
   __shared__ int s_cost[1024];
   __shared__ int s_prep[32];
   __shared__ int4 s_src[NW][2][16];
   __shared__ int4 s_out[NW][16];
-  __shared__ CostCol s_col[NW][2][80];
+  __shared__ AffCol s_col[NW][2][80];
   __shared__ int s_part[NW];
   __shared__ int s_pair, s_fin;
   const int tid = threadIdx.x, lane = tid & 63;
@@ -1268,16 +1588,7 @@ __global__ __launch_bounds__(64 * kCostWaves) void k_affine_cost_mw(AffCostArgs 
     int dV = kHigh, dCB = kHigh, dH = kHigh, dED = kHigh, lH = kHigh, lCB = kHigh;
     int oV = kHigh, oCB = kHigh, oH = kHigh, oED = kHigh;
     auto col_rec = [&](int j) __attribute__((always_inline)) {
-      CostCol c{0, 0, 0, 0};
-      if ((unsigned)j <= (unsigned)lenj) {
-        const int jc = sb[j], jp = j > 0 ? sb[j - 1] : sb[0];
-        const int gr = s_prep[jc];
-        c.go = has_gap_opening(j, jp, jc, go);
-        c.ext = (j != 1 && (jp & kGap) && !(jc & kGap)) ? c.go + gr : gr;
-        c.open = c.go + gr;
-        c.sym = ((jc & 15) << 2) | ((jc >> 4) & 1) | ((jp & kGap) ? 0 : 2);
-      }
-      return c;
+      return aff_col(sb, lenj, j, go, s_prep);
     };
     auto enter = [&]() {
       i = 1 + (b << 6) + lane;
@@ -1307,19 +1618,19 @@ __global__ __launch_bounds__(64 * kCostWaves) void k_affine_cost_mw(AffCostArgs 
         const int m = qb - P * b, s0 = m << 4, buf = m & 1;
         const bool more = m + 1 < nblk;
         int4 nsrc = make_int4(0, 0, 0, 0);
-        CostCol nc0{0, 0, 0, 0}, nc1{0, 0, 0, 0};
+        AffCol nc0{0, 0, 0, 0}, nc1{0, 0, 0, 0};
         if (more) {
           if (lane < 16) nsrc = rin[s0 + 16 + lane];
           nc0 = col_rec(s0 + 16 - 63 + lane);
           if (lane < 16) nc1 = col_rec(s0 + 16 + 1 + lane);
         }
-        const CostCol* const cw = &s_col[w][buf][63 - lane];
+        const AffCol* const cw = &s_col[w][buf][63 - lane];
         // every lane past column 0 and before the last one for all 16 steps
         const bool inner = s0 >= 64 && s0 + 15 <= lenj - 1;
         auto step = [&](const int u, auto edge_t) __attribute__((always_inline)) {
           constexpr bool kEdge = decltype(edge_t)::value;
           const int j = s0 + u - lane;
-          const CostCol c = cw[u];
+          const AffCol c = cw[u];
           const int4 src = s_src[w][buf][u];
           const int uV = wave_shr1(oV, src.x);
           const int uCB = wave_shr1(oCB, src.y);
@@ -1397,9 +1708,5 @@ __global__ __launch_bounds__(64 * kCostWaves) void k_affine_cost_mw(AffCostArgs 
     __syncthreads();
   }
 }
-
-template __global__ void k_affine_fill<true, false>(AffFillArgs);
-template __global__ void k_affine_fill<true, true>(AffFillArgs);
-template __global__ void k_affine_fill<false, false>(AffFillArgs);
 
 }  // namespace poyhip

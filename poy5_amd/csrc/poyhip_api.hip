@@ -459,6 +459,23 @@ hipError_t launch_linear_fill(poyhip_ctx* c, const LinFillArgs& A0, bool dm, int
   return hipGetLastError();
 }
 
+// The affine fill of A.pt's pairs with gap-bit symbols, on at most `slots`
+// workspaces.  Wavefronts per pair: as many as leave every pair of the launch
+// resident at 16 wavefronts a CU.  More shorten the longest pair (256 pairs
+// of 3,000 symbols: 20.5, 13.3, 11.1 ms on 1, 2, 4; 2,048 of 200-2,000: 25.3,
+// 18.4, 17.4), but narrow rounds leave them waiting, which costs once pairs
+// queue (2,048 pairs of 600: 3.3, 3.3, 5.2 ms; 8,192 of 300: 4.4, 5.7, 9.2).
+hipError_t launch_affine_general(poyhip_ctx* c, const AffFillArgs& A, int slots, hipStream_t st) {
+  const int n = A.pt.n, cus = c->num_cus;
+  if (n > 8 * cus)
+    hipLaunchKernelGGL(k_affine_fill_gen<1>, dim3(std::min(slots, 16 * cus)), dim3(64), 0, st, A);
+  else if (n > 4 * cus)
+    hipLaunchKernelGGL(k_affine_fill_gen<2>, dim3(std::min(slots, 8 * cus)), dim3(128), 0, st, A);
+  else
+    hipLaunchKernelGGL(k_affine_fill_gen<4>, dim3(std::min(slots, 4 * cus)), dim3(256), 0, st, A);
+  return hipGetLastError();
+}
+
 int run_linear_one(poyhip_ctx* c, const uint8_t* s1, int l1, const uint8_t* s2, int l2,
                    int deltawh, int prio, bool backtrace, PairResult* out_res,
                    std::vector<uint8_t>* outblk, int outlen[4], const int* limit = nullptr) {
@@ -1033,8 +1050,7 @@ int poyhip_align_affine_3(poyhip_ctx* c, const uint8_t* si, int li, const uint8_
   for (int k = 1; k < li; k++) any |= si[k];
   for (int k = 1; k < lj; k++) any |= sj[k];
   if (any & kGap) {
-    hipLaunchKernelGGL((k_affine_fill<true, false>), dim3(1), dim3(64), 0, c->stream, A);
-    HIPCHK(c, hipGetLastError());
+    HIPCHK(c, launch_affine_general(c, A, 1, c->stream));
     AffBtArgs B;
     B.pt = t;
     B.cm = c->d_cm;
@@ -1048,7 +1064,7 @@ int poyhip_align_affine_3(poyhip_ctx* c, const uint8_t* si, int li, const uint8_
     // the gap-free kernel runs the backtrace after the fill
     A.out = dout;
     A.outlen = doutlen;
-    hipLaunchKernelGGL((k_affine_fill<true, true>), dim3(1), dim3(64), 0, c->stream, A);
+    hipLaunchKernelGGL(k_affine_fill, dim3(1), dim3(64), 0, c->stream, A);
   }
   HIPCHK(c, hipGetLastError());
   const size_t back = kResBytes + outb;
@@ -1120,8 +1136,7 @@ int poyhip_align_affine_3_noalloc(poyhip_ctx* c, const uint8_t* si, int li, cons
   for (int k = 1; k < li; k++) any |= si[k];
   for (int k = 1; k < lj; k++) any |= sj[k];
   if (any & kGap) {
-    hipLaunchKernelGGL((k_affine_fill<true, false>), dim3(1), dim3(64), 0, c->stream, A);
-    HIPCHK(c, hipGetLastError());
+    HIPCHK(c, launch_affine_general(c, A, 1, c->stream));
     AffBtArgs B;
     B.pt = t;
     B.cm = c->d_cm;
@@ -1134,7 +1149,7 @@ int poyhip_align_affine_3_noalloc(poyhip_ctx* c, const uint8_t* si, int li, cons
   } else {
     A.out = dout;
     A.outlen = doutlen;
-    hipLaunchKernelGGL((k_affine_fill<true, true>), dim3(1), dim3(64), 0, c->stream, A);
+    hipLaunchKernelGGL(k_affine_fill, dim3(1), dim3(64), 0, c->stream, A);
   }
   HIPCHK(c, hipGetLastError());
   // result header first, then each output region straight into the
@@ -1461,9 +1476,9 @@ int batch_enqueue(poyhip_batch* b, const uint8_t* blob, const int64_t* off1, con
           A.out = d_out;  // each pair's backtrace follows its fill
           A.outlen = d_outlen;
           A.counter = b->d_counters + 2 * k;
-          hipLaunchKernelGGL((k_affine_fill<true, true>), dim3(b->grid), dim3(64), 0, st, A);
+          hipLaunchKernelGGL(k_affine_fill, dim3(b->grid), dim3(64), 0, st, A);
           A.counter = b->d_counters + 2 * k + 1;
-          hipLaunchKernelGGL((k_affine_fill<true, false>), dim3(b->grid), dim3(64), 0, st, A);
+          HIPCHK(c, launch_affine_general(c, A, b->grid, st));
         }
         break;
       }

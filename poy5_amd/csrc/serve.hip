@@ -320,9 +320,9 @@ int srv_launch(poyhip_server* s, SrvSlot& sl) {
     // takes the pairs with gap-bit symbols
     A.out = sl.d_out;
     A.outlen = sl.d_outlen;
-    hipLaunchKernelGGL((k_affine_fill<true, true>), dim3(grid), dim3(64), 0, st, A);
+    hipLaunchKernelGGL(k_affine_fill, dim3(grid), dim3(64), 0, st, A);
     A.counter = sl.d_counters + 1;
-    hipLaunchKernelGGL((k_affine_fill<true, false>), dim3(grid), dim3(64), 0, st, A);
+    HIPCHK(c, launch_affine_general(c, A, grid, st));
     AffBtArgs B;
     B.pt = pt;
     B.cm = c->d_cm;
