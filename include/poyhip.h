@@ -352,10 +352,10 @@ int poyhip_union_merge_batch(poyhip_ctx *ctx, int n, const poyhip_union_job *d_j
  *                     schedule within its limits (default); 0: the plain
  *                     stripe loop
  *   LINEAR_WORKGROUP  when every cost entry fits 16 bits, 2: the linear
- *                     fill runs a workgroup of wavefronts per pair unless
- *                     the batch has at least 16 pairs per CU, which run one
- *                     wavefront each (default); 1: always a workgroup per
- *                     pair; 0: always one wavefront per pair
+ *                     fill sweeps anti-diagonals, on as many wavefronts per
+ *                     pair as the batch leaves room for (default); 1: stripes
+ *                     on a workgroup per pair; 0: stripes on one wavefront
+ *                     per pair
  *   CUBE_WORKGROUP    1: the 3D fill runs a workgroup per triple when its
  *                     keys fit (default); 0: one wavefront per triple
  * Results do not depend on the knobs.  get returns the value or

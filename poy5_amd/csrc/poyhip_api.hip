@@ -390,13 +390,21 @@ void launch_linear_wide(const LinFillArgs& A, bool dm, int grid, hipStream_t st)
 // A.ws_stride ints are available.  `diag` false keeps to the stripe fills.
 // Returns the launch error.
 //
-// The anti-diagonal fill comes first: in key form with one wavefront per pair
-// when the pairs alone fill the SIMDs, four when they do not and sixteen when
-// every pair can have a CU, in wide form with sixteen when value and count do
-// not fit a key.  Pairs it leaves (a
-// band wider than its lanes, a direction store larger than the stripe
-// layout's region) go through the sixteen-wavefront form, then the stripe
-// fill.
+// The anti-diagonal fill comes first.  In key form it takes sixteen
+// wavefronts per pair when every pair can have a CU, one when the pairs alone
+// fill the SIMDs, four between.  What is best depends on the band, which is
+// not known before, so the lines avoid the bad ends.  Pairs of 1,500 symbols
+// that differ by 3% and 25%, on 16 / 4 / 1 wavefronts: 256 pairs 0.58 / 0.42 /
+// 0.33 and 0.52 / 0.55 / 1.47 ms; 1,024 pairs 1.67 / 0.64 / 0.36 and 1.50 /
+// 0.86 / 2.06 ms; 256 pairs of 6,000 at 25% 3.2 / 8.7 / 4.2 ms; 2,048 pairs of
+// 3,000 at 8% 5.0 / 2.4 / 1.7 ms.  A line for short pairs alone did not pay:
+// 1,024 pairs of 600 alike at 3% and 25% take 0.31 / 0.19 and 0.30 / 0.31 ms on
+// 4 / 1, but mixed pairs of 300-700 0.39 and 0.46 ms.
+// The wide form, always on sixteen, is for values and counts that do
+// not fit a key (1,024 pairs of 600: 0.91 ms against 0.68 in key form).
+// Pairs it leaves (a band wider than its lanes, a direction store larger than
+// the stripe layout's region) go through the sixteen-wavefront form, then the
+// stripe fill.
 hipError_t launch_linear_fill(poyhip_ctx* c, const LinFillArgs& A0, bool dm, int slots,
                               int64_t max_sum, bool diag, hipStream_t st) {
   LinFillArgs A = A0;

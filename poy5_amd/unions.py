@@ -122,8 +122,8 @@ def pack_level(merges):
 
 class Level:
     """A packed level resident on the device, run as one launch.  The jobs
-    are laid out longest walk first: a wavefront runs as long as its longest
-    merge, so merges of similar length share wavefronts."""
+    are laid out longest walk first: a merge has a wavefront of its own, and
+    the level ends with its last one."""
 
     def __init__(self, ctx: Context, merges, device="cuda"):
         self.ctx = ctx
